@@ -111,6 +111,18 @@ PQ_HIDDEN void launch_rotate_quant_group(const void* x, int x_dtype, const RotGr
                                          int krot, unsigned flags, hipStream_t stream,
                                          const NormArgs* norm = nullptr);
 
+// launch_rotate_quant_group and the plain / MXFP4 rows of pq_rotate_rows
+// (grp.count = 1) for one input dtype (pq_rows.h).
+#define PQ_ROWS_DECL(dt)                                                                                              \
+  PQ_HIDDEN void launch_rows_##dt(const void* x, const RotGroup& grp, int64_t rows, int h, int krot, unsigned flags,  \
+                                  hipStream_t stream, const NormArgs* norm);                                          \
+  PQ_HIDDEN void launch_plain_rows_##dt(const void* x, const RotGroup& grp, int64_t rows, int h, int krot,            \
+                                        int out_mode, hipStream_t stream);
+PQ_ROWS_DECL(f32)
+PQ_ROWS_DECL(f16)
+PQ_ROWS_DECL(bf16)
+#undef PQ_ROWS_DECL
+
 // Decode GEMM whose A operand is quantized in the kernel from launch_rotate_split's
 // output: token scale = max over the row's gmax / 127.  Returns false when m or
 // the LDS image of A (m x (k + 16) bytes) is out of range.
