@@ -114,6 +114,21 @@ __device__ __forceinline__ void store_f16xn(uint16_t* p, const float (&v)[N]) {
 }
 
 // ---------------------------------------------------------------------------
+// Tiled int8 activations, m * k bytes: row blocks of 16 rows, each
+// [G][2][4][r][16] bytes with r its rows (16; m % 16 of them in a ragged last
+// block, so nothing is padded).  Part (g, p, j, c) holds codes
+// 128 g + 32 j + 16 p .. + 15 of the block's row c: the order in which lane
+// 16 j + c of v_mfma_i32_16x16x64_i8 takes its two operands of a group, so
+// that a fragment of a full block is one contiguous 1 KB load.
+// ---------------------------------------------------------------------------
+__host__ __device__ __forceinline__ int64_t a_tile_offset(int64_t row, int k, int64_t m, int G) {
+  const int64_t r0 = row & ~static_cast<int64_t>(15);
+  const int r = m - r0 < 16 ? static_cast<int>(m - r0) : 16;
+  return r0 * G * 128 + ((k >> 7) * 128 + ((k >> 4) & 1) * 64 + ((k >> 5) & 3) * 16) * r +
+         static_cast<int>(row - r0) * 16 + (k & 15);
+}
+
+// ---------------------------------------------------------------------------
 // int4 weight unpacking (layout in pq_gemm.hip): a dword of 8 codes -> two
 // dwords of 4 signed bytes (q - z).  Every byte stays in [113, 143] before the
 // xor, so no carry crosses a byte; the xor maps 128 + d to two's complement d.

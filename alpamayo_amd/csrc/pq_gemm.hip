@@ -500,7 +500,11 @@ __device__ __forceinline__ void wait_groups(int ahead) {
   }
 }
 
-template <int BM, int BN, int WM, int WN, bool PARTIALS, int ST = kPfStages, bool TP = false>
+// CLS > 1: the sum over the groups is taken in CLS chains, chain c over groups
+// c, c + CLS, ..., then ((chain 0 + chain 1) + ...): the order in which the
+// mid-size GEMM adds the partial sums of CLS waves, so that a row's outputs
+// have the same bits on either kernel.  One more set of accumulators.
+template <int BM, int BN, int WM, int WN, bool PARTIALS, int ST = kPfStages, bool TP = false, int CLS = 1>
 __global__ __launch_bounds__(WM * WN * 64) void gemm_prefill(
     const pq::GemmGroup grp, int bias_dtype, int y_dtype, int M, int K) {
   constexpr int NW = WM * WN;
@@ -592,11 +596,11 @@ __global__ __launch_bounds__(WM * WN * 64) void gemm_prefill(
 #pragma unroll
   for (int tn = 0; tn < TN; ++tn) bcol[tn] = wn * (BN / WN) + tn * 32 + r32;
 
-  // Matrix work of group g from its stage.  The loads of group ig (= g + 2)
+  // Matrix work of group g from its stage.  The loads of step ig (two ahead, group gi)
   // are issued after the first two k-steps' MFMAs: issued at the top of the
   // group, right after the barrier, all waves' copies queue up at once in
   // the load path while no MFMA is in flight.
-  auto compute = [&](int stage, int g, int ig) {
+  auto compute = [&](int stage, int g, int ig, int gi) {
     const uint8_t* As = smem + stage * STAGE;
     const uint8_t* Bs = As + A_BYTES;
     const uint32_t* Ms = reinterpret_cast<const uint32_t*>(Bs + B_BYTES);
@@ -632,7 +636,7 @@ __global__ __launch_bounds__(WM * WN * 64) void gemm_prefill(
 #pragma unroll
         for (int tn = 0; tn < TN; ++tn)
           T[tm][tn] = __builtin_amdgcn_mfma_i32_32x32x32_i8(a[tm], b[tn], T[tm][tn], 0, 0, 0);
-      if (i == 1 && ig < G) issue(ig, ig % ST);
+      if (i == 1 && ig < G) issue(gi, ig % ST);
     }
     if constexpr (PARTIALS) {
 #pragma unroll
@@ -668,7 +672,7 @@ __global__ __launch_bounds__(WM * WN * 64) void gemm_prefill(
     const int n = bn * BN + bcol[tn];
     if (m < M && n < N) partials[(m * G + g) * N + n] = val;
   };
-  auto compute_tp = [&](int stage, int g, int ig) {
+  auto compute_tp = [&](int stage, int g, int ig, int gi) {
     static_assert(!TP || TM % 2 == 0, "tiles in pairs");
     const uint8_t* As = smem + stage * STAGE;
     const uint8_t* Bs = As + A_BYTES;
@@ -735,7 +739,7 @@ __global__ __launch_bounds__(WM * WN * 64) void gemm_prefill(
           __builtin_amdgcn_sched_group_barrier(0x002, 8, 0);   // eight VALU
         }
       }
-      if (p == 0 && ig < G) issue(ig, ig % ST);
+      if (p == 0 && ig < G) issue(gi, ig % ST);
     }
     constexpr int LP = (TM / 2 - 1) & 1;
 #pragma unroll
@@ -761,16 +765,48 @@ __global__ __launch_bounds__(WM * WN * 64) void gemm_prefill(
     lds_copy4(xs + min(bm * BM + r, M - 1), lds0 + ST * STAGE + wave * 256);
   }
   static_assert(LOADS * (ST - 2) < 64, "vmcnt range");
+  // Step i computes the i-th group of the order: ascending, or chain by chain.
+  auto after = [&](int g) { return CLS == 1 || g + CLS < G ? g + CLS : g % CLS + 1; };
+  float tot[CLS > 1 ? TM : 1][TN][16];
+  int gq = 0;   // the next group to copy
 #pragma unroll
   for (int q = 0; q < ST - 1; ++q)
-    if (q < G) issue(q, q);
-  for (int g = 0; g < G; ++g) {
-    wait_groups<LOADS, ST - 2>(min(G - 1 - g, ST - 2));
+    if (q < G) {
+      issue(gq, q);
+      gq = after(gq);
+    }
+  int g = 0;
+  for (int i = 0; i < G; ++i) {
+    wait_groups<LOADS, ST - 2>(min(G - 1 - i, ST - 2));
     __builtin_amdgcn_s_barrier();
-    if constexpr (TP) compute_tp(g % ST, g, g + ST - 1);
-    else compute(g % ST, g, g + ST - 1);
+    if constexpr (TP) compute_tp(i % ST, g, i + ST - 1, gq);
+    else compute(i % ST, g, i + ST - 1, gq);
+    if constexpr (CLS > 1) {
+      if (g + CLS >= G) {   // the chain's last group
+        const bool first = g % CLS == 0;
+#pragma unroll
+        for (int tm = 0; tm < TM; ++tm)
+#pragma unroll
+          for (int tn = 0; tn < TN; ++tn)
+#pragma unroll
+            for (int v = 0; v < 16; ++v) {
+              tot[tm][tn][v] = first ? acc[tm][tn][v] : tot[tm][tn][v] + acc[tm][tn][v];
+              acc[tm][tn][v] = 0.0f;
+            }
+      }
+    }
+    g = after(g);
+    gq = after(gq);
   }
   if constexpr (PARTIALS) return;
+  if constexpr (CLS > 1) {
+#pragma unroll
+    for (int tm = 0; tm < TM; ++tm)
+#pragma unroll
+      for (int tn = 0; tn < TN; ++tn)
+#pragma unroll
+        for (int v = 0; v < 16; ++v) acc[tm][tn][v] = tot[tm][tn][v];
+  }
 
   // Output, one 32-row slice per wave row at a time (WM*32 rows of the
   // tile): the waves write their values in the output type to LDS, then
@@ -839,14 +875,14 @@ __global__ __launch_bounds__(WM * WN * 64) void gemm_prefill(
   else emit(std::integral_constant<int, PQ_BF16>{});
 }
 
-template <int BM, int BN, int WM, int WN, bool PARTIALS, int ST = kPfStages, bool TP = false>
+template <int BM, int BN, int WM, int WN, bool PARTIALS, int ST = kPfStages, bool TP = false, int CLS = 1>
 void launch_prefill_t(pq::GemmGroup grp, int bias_dtype, int y_dtype, int M, int K,
                       hipStream_t stream) {
   constexpr int STAGE = BM * 128 + (BN / 16) * kPfBStride + BN * 4;
   grp.first[0] = 0;
   for (int i = 0; i < grp.count; ++i) grp.first[i + 1] = grp.first[i] + (grp.mem[i].n + BN - 1) / BN;
   const unsigned grid = static_cast<unsigned>(((M + BM - 1) / BM) * grp.first[grp.count]);
-  gemm_prefill<BM, BN, WM, WN, PARTIALS, ST, TP><<<grid, WM * WN * 64, ST * STAGE + BM * 4, stream>>>(
+  gemm_prefill<BM, BN, WM, WN, PARTIALS, ST, TP, CLS><<<grid, WM * WN * 64, ST * STAGE + BM * 4, stream>>>(
       grp, bias_dtype, y_dtype, M, K);
 }
 
@@ -1055,6 +1091,12 @@ int check_gemm_args(const char* who, int64_t m, int64_t n, int64_t k, int group_
 namespace pq {
 bool gemm_rotated_supported(int64_t m, int64_t k) {
   return m >= 1 && m <= kSkinnyRows && k % 128 == 0 && k <= 16384 && m * (k + 16) <= 80 * 1024;
+}
+
+void launch_gemm_chains(const GemmGroup& grp, int chains, int bias_dtype, int y_dtype, int m, int k,
+                        hipStream_t stream) {
+  if (chains == 8) launch_prefill_t<128, 256, 1, 8, false, kPfStages, true, 8>(grp, bias_dtype, y_dtype, m, k, stream);
+  else launch_prefill_t<128, 256, 1, 8, false, kPfStages, true, 4>(grp, bias_dtype, y_dtype, m, k, stream);
 }
 
 void launch_gemm_group(GemmGroup grp, int aq, int bias_dtype, int y_dtype, int m, int k, hipStream_t stream) {

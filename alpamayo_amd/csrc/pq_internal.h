@@ -54,6 +54,7 @@ struct RotMember {
 struct RotGroup {
   RotMember mem[kMaxGroup];
   int count;
+  int tiled;   // row kernel: rows m of the tiled order (pqd::a_tile_offset) for the int8 codes; 0: row-major
 };
 
 // Per-token int8 quantization of a split rotation's output (launch_quant_split):
@@ -67,6 +68,7 @@ struct QuantMember {
 struct QuantGroup {
   QuantMember mem[kMaxGroup];
   int count;
+  int tiled;   // rows m of the tiled order (pqd::a_tile_offset) for xq; 0: row-major
 };
 
 // Rows per launch of the split rotation (and rows the rotated GEMM accepts).
@@ -136,6 +138,27 @@ PQ_HIDDEN void launch_gemm_group(GemmGroup grp, int aq, int bias_dtype, int y_dt
 // their partials form: each member's int32 partials (and, for aq != 0, its
 // A image and token scales) go to the member's partials / a_out / as_out.
 PQ_HIDDEN void launch_gemm_group_partials(GemmGroup grp, int aq, int m, int k, hipStream_t stream);
+
+// The GEMM of a group on tiled int8 codes (xq in the order of
+// pqd::a_tile_offset): whether it is the one
+// to run for m rows and n_total output columns, and its launches.
+//
+// From kMidFixedRows + 1 rows on, a row's outputs must not depend on which
+// linears share its launch (a group returns the bits its members return when
+// called one by one), so the order of the sum over K is fixed by m: 8 chains
+// up to 128 rows, 4 above (gemm_chains), whatever the number of columns; a
+// launch too wide for the mid-size GEMM then runs the prefill tiles with the
+// same chains (launch_gemm_chains, row-major codes).
+constexpr int kMidFixedRows = 64, kMidMaxRows = 512;
+enum class MidGemm { kNone, kTiled, kChains };
+PQ_HIDDEN MidGemm gemm_mid_choice(const GemmGroup& grp, int64_t m, int64_t k);
+constexpr int gemm_chains(int64_t m) { return m <= 128 ? 8 : 4; }
+PQ_HIDDEN void launch_gemm_chains(const GemmGroup& grp, int chains, int bias_dtype, int y_dtype, int m, int k,
+                                  hipStream_t stream);
+PQ_HIDDEN void launch_gemm_mid(const GemmGroup& grp, int bias_dtype, int y_dtype, int m, int k, hipStream_t stream);
+PQ_HIDDEN void launch_gemm_mid_partials(const GemmGroup& grp, int m, int k, hipStream_t stream);
+// Row-major copy [m][k] of tiled codes.
+PQ_HIDDEN void launch_untile_a(const int8_t* tiled, int8_t* out, int m, int k, hipStream_t stream);
 
 }  // namespace pq
 

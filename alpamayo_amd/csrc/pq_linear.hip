@@ -190,6 +190,10 @@ int linear_group(const char* who, const void* x, int x_dtype, const pq_linear_me
                    static_cast<int>(mb.n)};
     }
   }
+  // The mid-size GEMM reads the int8 codes in the tiled order, which the quant launches then write.
+  const pq::MidGemm mid = path != Path::kSplit ? pq::gemm_mid_choice(gg, m, k) : pq::MidGemm::kNone;
+  const bool tiled = mid == pq::MidGemm::kTiled;
+  rg.tiled = qg.tiled = tiled ? M : 0;
   int st = PQ_OK;
   if (stage == 2) {
     // the GEMM alone, from the workspace stage 1 filled
@@ -207,6 +211,11 @@ int linear_group(const char* who, const void* x, int x_dtype, const pq_linear_me
   }
   if (st != PQ_OK || stage == 1) return st;
   const int aq = path == Path::kSplit ? (mat16 ? 1 : 2) : 0;
+  if (probe == nullptr && mid != pq::MidGemm::kNone) {
+    if (tiled) pq::launch_gemm_mid(gg, bias_dtype, y_dtype, M, K, s);
+    else pq::launch_gemm_chains(gg, pq::gemm_chains(M), bias_dtype, y_dtype, M, K, s);
+    return pq::launch_status("linear GEMM launch");
+  }
   if (probe == nullptr) {
     pq::launch_gemm_group(gg, aq, bias_dtype, y_dtype, M, K, s);
     return pq::launch_status("linear GEMM launch");
@@ -223,14 +232,17 @@ int linear_group(const char* who, const void* x, int x_dtype, const pq_linear_me
     gg.mem[i].bias = nullptr;
     col0 += members[i].n;
     if (path != Path::kSplit) {
-      hipError_t e = hipMemcpyAsync(gg.mem[i].a_out, gg.mem[i].xq, static_cast<size_t>(m * k), hipMemcpyDeviceToDevice, s);
+      hipError_t e = hipSuccess;
+      if (tiled) pq::launch_untile_a(gg.mem[i].xq, gg.mem[i].a_out, M, K, s);
+      else e = hipMemcpyAsync(gg.mem[i].a_out, gg.mem[i].xq, static_cast<size_t>(m * k), hipMemcpyDeviceToDevice, s);
       if (e == hipSuccess)
         e = hipMemcpyAsync(gg.mem[i].as_out, gg.mem[i].xs, static_cast<size_t>(m) * sizeof(float),
                            hipMemcpyDeviceToDevice, s);
       PQ_REQUIRE(e == hipSuccess, PQ_ERR_HIP, "%s: copy of member %d's A operand: %s", who, i, hipGetErrorString(e));
     }
   }
-  pq::launch_gemm_group_partials(gg, aq, M, K, s);
+  if (tiled) pq::launch_gemm_mid_partials(gg, M, K, s);
+  else pq::launch_gemm_group_partials(gg, aq, M, K, s);
   return pq::launch_status("linear GEMM partials launch");
 }
 

@@ -331,7 +331,7 @@ __global__ __launch_bounds__(256) void quant_split_kernel(const pq::QuantGroup g
     q.x = pqd::quant4(va.x, va.y, va.z, va.w, inv);
     q.y = pqd::quant4(vb.x, vb.y, vb.z, vb.w, inv);
   }
-  *reinterpret_cast<uint2*>(mb.xq + o) = q;
+  *reinterpret_cast<uint2*>(mb.xq + (grp.tiled ? pqd::a_tile_offset(row, c8, grp.tiled, G) : o)) = q;
   if (c8 == 0) mb.xscale[row] = am / 127.0f;
 }
 

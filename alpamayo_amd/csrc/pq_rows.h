@@ -379,7 +379,7 @@ __global__ __launch_bounds__(kRQWaves * 64) void rotate_quant_kernel(const void*
             const int i = k * RB + r;
             c[k] = pqd::quant_scaled(pqd::mul_f16(d[i >> 1], (i & 1) != 0, inv));
           }
-          *reinterpret_cast<uint2*>(xq + ro) =
+          *reinterpret_cast<uint2*>(xq + (grp.tiled ? pqd::a_tile_offset(row0 + r, c8, grp.tiled, G) : ro)) =
               make_uint2(pqd::pack4(c[0], c[1], c[2], c[3]), pqd::pack4(c[4], c[5], c[6], c[7]));
         }
       }
@@ -408,7 +408,7 @@ __global__ __launch_bounds__(kRQWaves * 64) void rotate_quant_kernel(const void*
         uint2 o;
         o.x = quant4(f[0], f[1], f[2], f[3], inv);
         o.y = quant4(f[4], f[5], f[6], f[7], inv);
-        *reinterpret_cast<uint2*>(xq + (row0 + r) * h + c8) = o;
+        *reinterpret_cast<uint2*>(xq + (grp.tiled ? pqd::a_tile_offset(row0 + r, c8, grp.tiled, G) : (row0 + r) * h + c8)) = o;
       }
     }
   }

@@ -1,0 +1,65 @@
+"""The GEMM on tiled int8 activations (17 rows up to a few hundred) behind the W4A8 linear entry points, at the edges
+of its row blocks, column units and K splits: the codes and int32 partials as in test_gpu_intermediates.py, and the
+float32 outputs against float64 sums of the same codes.
+
+Bound of the outputs: a sum of G float32 terms s_g * P_g (P_g exact in float32, one fma each), in any order, then one
+product with the token scale and one add of the bias, is off by at most (G + 3) 2^-24 sum_g |s_g P_g| * xscale + 2^-24 |y|.
+"""
+
+import zlib
+
+import numpy as np
+import pytest
+import torch
+
+import alpamayo_amd  # noqa: F401
+from alpamayo_amd import workloads
+from tests.gpu_util import to_np
+from tests.test_gpu_group import _members
+from tests.test_gpu_intermediates import _check, _run
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("M,K,ns,flags", [
+    (17, 1024, (16,), (True, True)),             # one wave per group of K, one ragged column unit
+    (31, 1152, (4096,), (True, True)),           # nine groups over eight waves, one column tile per wave
+    (32, 4096, (4112, 48), (True, True)),        # odd column tiles in both members
+    (33, 4096, (4096, 1024, 1024), (True, True)),
+    (47, 12288, (4096,), (True, True)),
+    (64, 1408, (8192, 8208), (True, True)),
+    (65, 4096, (4096,), (True, True)),           # first size on the row rotate+quant kernel
+    (97, 2048, (1040, 80), (False, False)),      # float32 rows
+    (128, 4096, (4096, 1024, 1024), (True, True)),
+    (200, 4224, (4096,), (True, True)),          # 33 groups: uneven K splits
+    (255, 1024, (5120,), (True, True)),
+    (511, 1024, (1040,), (True, True)),          # the most rows it takes, less one
+    (160, 1152, (12288, 12304), (True, True)),   # too wide: the prefill tiles in four chains of K
+    (113, 1408, (24576,), (True, True)),         # in eight chains
+])
+def test_tiled_gemm(M, K, ns, flags):
+    print(f"tiled GEMM M={M} K={K} ns={ns} flags={flags}", flush=True)
+    krot = 8
+    mbs = _members(ns, K, krot, zlib.crc32(f"mid{ns}-{K}".encode()), with_bias=True)
+    x = workloads.activations(M, K, workloads.generator(7 * M + K)).cuda()
+    codes, xscale, parts, _, _ = _run(mbs, x, krot, flags)
+    rows = np.unique(np.concatenate([np.arange(0, M, max(1, M // 24)), np.arange(max(0, M - 17), M)]))
+    _check(mbs, to_np(x), codes, xscale, parts, flags, rows=rows)
+    args = ([m["rot_idx"] for m in mbs], [m["rot_cs"] for m in mbs], [m["scales"] for m in mbs], krot,
+            [m["wp"] for m in mbs], [m["wm"] for m in mbs], [m["bias"] for m in mbs], *flags)
+    ys = torch.ops.paroquant.w4a8_linear_group(x, *args, torch.float32)
+    y16 = torch.ops.paroquant.w4a8_linear_group(x, *args, torch.bfloat16)
+    for i, (mb, y) in enumerate(zip(mbs, ys)):
+        sc = (mb["wm"].cpu().numpy().view(np.uint32) & 0xFFFF).astype(np.uint16).view(np.float16)   # [N/16, G, 16]
+        s = sc.transpose(1, 0, 2).reshape(K // 128, -1).astype(np.float64)
+        terms = to_np(parts[i]).astype(np.float64) * s[None]
+        xs = to_np(xscale[i]).astype(np.float64)[:, None]
+        b = to_np(mb["bias"].float()).astype(np.float64) if mb["bias"] is not None else np.zeros(1)
+        ref = terms.sum(1) * xs + b
+        bound = (K // 128 + 3) * 2.0 ** -24 * np.abs(terms).sum(1) * xs + 2.0 ** -23 * (np.abs(ref) + np.abs(b))
+        assert np.all(np.abs(to_np(y).astype(np.float64) - ref) <= bound)
+        if M > 64:   # the bits of the member called by itself, whichever kernel that call takes
+            single = torch.ops.paroquant.w4a8_linear(x, *(a[i] for a in args[:3]), krot, *(a[i] for a in args[4:7]), *flags,
+                                                     torch.float32)
+            assert torch.equal(y, single)
+        assert torch.equal(y16[i].view(torch.int16), y.to(torch.bfloat16).view(torch.int16))
