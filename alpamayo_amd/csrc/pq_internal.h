@@ -94,6 +94,10 @@ struct NormArgs {
   int mode;
 };
 
+// The prologue arguments of the fused group entry points, checked.
+PQ_HIDDEN int prologue_args(const char* who, const void* x2, const void* norm_weight, float eps, int mode,
+                            void* h_out, void* sum_out, int x_dtype, int64_t m, NormArgs* out);
+
 // Rotation of m <= kSplitMaxRows rows with one wave per 128-channel group,
 // for every member of the group: xr [m][h] rotated values (fp16 when flags
 // has PQ_RQ_MATERIALIZE_FP16, else fp32) and gmax [m][h/128] the absmax of

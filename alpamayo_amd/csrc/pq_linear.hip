@@ -246,9 +246,12 @@ int linear_group(const char* who, const void* x, int x_dtype, const pq_linear_me
   return pq::launch_status("linear GEMM partials launch");
 }
 
+}  // namespace
+
+namespace pq {
 // The prologue arguments of the fused group entry points, checked.
 int prologue_args(const char* who, const void* x2, const void* norm_weight, float eps, int mode, void* h_out,
-                  void* sum_out, int x_dtype, int64_t m, pq::NormArgs* out) {
+                  void* sum_out, int x_dtype, int64_t m, NormArgs* out) {
   PQ_REQUIRE(mode == PQ_PRO_RMSNORM || mode == PQ_PRO_ADD || mode == PQ_PRO_SWIGLU, PQ_ERR_ARG, "%s: mode %d", who,
              mode);
   PQ_REQUIRE(x_dtype == PQ_F32 || x_dtype == PQ_F16 || x_dtype == PQ_BF16, PQ_ERR_UNSUPPORTED, "%s: x dtype code %d",
@@ -256,14 +259,14 @@ int prologue_args(const char* who, const void* x2, const void* norm_weight, floa
   if (mode == PQ_PRO_RMSNORM)
     PQ_REQUIRE(eps >= 0.0f && eps < 1.0f, PQ_ERR_ARG, "%s: eps=%g must be in [0, 1)", who, static_cast<double>(eps));
   if (m > 0) {
-    const size_t es = static_cast<size_t>(pq::dtype_size(x_dtype));
+    const size_t es = static_cast<size_t>(dtype_size(x_dtype));
     if (mode == PQ_PRO_RMSNORM)
-      PQ_REQUIRE(norm_weight != nullptr && pq::aligned_to(norm_weight, es), PQ_ERR_ARG,
+      PQ_REQUIRE(norm_weight != nullptr && aligned_to(norm_weight, es), PQ_ERR_ARG,
                  "%s: norm_weight must be non-null and aligned to its dtype", who);
     else
       PQ_REQUIRE(x2 != nullptr, PQ_ERR_ARG, "%s: mode %d needs x2 (the residual / up rows)", who, mode);
-    PQ_REQUIRE(x2 == nullptr || pq::aligned_to(x2, 16), PQ_ERR_ARG, "%s: x2 (the residual or up rows) must be 16-byte aligned", who);
-    PQ_REQUIRE((h_out == nullptr || pq::aligned_to(h_out, es)) && (sum_out == nullptr || pq::aligned_to(sum_out, es)),
+    PQ_REQUIRE(x2 == nullptr || aligned_to(x2, 16), PQ_ERR_ARG, "%s: x2 (the residual or up rows) must be 16-byte aligned", who);
+    PQ_REQUIRE((h_out == nullptr || aligned_to(h_out, es)) && (sum_out == nullptr || aligned_to(sum_out, es)),
                PQ_ERR_ARG, "%s: h_out and sum_out must be aligned to x's dtype", who);
     PQ_REQUIRE(sum_out == nullptr || (mode != PQ_PRO_SWIGLU && x2 != nullptr), PQ_ERR_ARG,
                "%s: sum_out needs a residual (and no SwiGLU)", who);
@@ -272,8 +275,7 @@ int prologue_args(const char* who, const void* x2, const void* norm_weight, floa
   *out = {x2, mode == PQ_PRO_RMSNORM ? norm_weight : nullptr, h_out, sum_out, eps, mode};
   return PQ_OK;
 }
-
-}  // namespace
+}  // namespace pq
 
 extern "C" size_t pq_w4a8_linear_workspace_size(int64_t m, int64_t n, int64_t k, int krot) {
   (void)krot;
@@ -360,7 +362,7 @@ extern "C" int pq_w4a8_linear_group_fused(const void* x, const void* x2, const v
                                           unsigned flags, void* workspace, size_t workspace_bytes, void* stream) {
   const char* who = "pq_w4a8_linear_group_fused";
   pq::NormArgs pro{};
-  const int st = prologue_args(who, x2, norm_weight, eps, mode, h_out, sum_out, x_dtype, m, &pro);
+  const int st = pq::prologue_args(who, x2, norm_weight, eps, mode, h_out, sum_out, x_dtype, m, &pro);
   if (st != PQ_OK) return st;
   return linear_group(who, x, x_dtype, members, count, bias_dtype, y_dtype, m, k, krot, flags, workspace,
                       workspace_bytes, static_cast<hipStream_t>(stream), &pro);
@@ -375,7 +377,7 @@ extern "C" int pq_w4a8_linear_group_stage(int stage, const void* x, const void* 
   PQ_REQUIRE(stage == 1 || stage == 2, PQ_ERR_ARG, "%s: stage %d (1 = rotation launches, 2 = GEMM)", who, stage);
   pq::NormArgs pro{};
   if (stage == 1 && mode != 0) {
-    const int st = prologue_args(who, x2, norm_weight, eps, mode, h_out, sum_out, x_dtype, m, &pro);
+    const int st = pq::prologue_args(who, x2, norm_weight, eps, mode, h_out, sum_out, x_dtype, m, &pro);
     if (st != PQ_OK) return st;
   }
   return linear_group(who, x, x_dtype, members, count, bias_dtype, y_dtype, m, k, krot, flags, workspace,
@@ -391,7 +393,7 @@ extern "C" int pq_w4a8_linear_group_intermediates(const void* x, const void* x2,
   const char* who = "pq_w4a8_linear_group_intermediates";
   pq::NormArgs pro{};
   if (mode != 0) {
-    const int st = prologue_args(who, x2, norm_weight, eps, mode, h_out, sum_out, x_dtype, m, &pro);
+    const int st = pq::prologue_args(who, x2, norm_weight, eps, mode, h_out, sum_out, x_dtype, m, &pro);
     if (st != PQ_OK) return st;
   }
   const Probe probe = {codes, xscale, partials};

@@ -547,7 +547,7 @@ namespace {
 // sizes.
 int w16_linear_group(const char* who, const void* x, int x_dtype, const pq_linear_member* members, int count,
                      int bias_dtype, int y_dtype, int64_t m, int64_t k, int krot, unsigned flags, void* workspace,
-                     size_t workspace_bytes, hipStream_t s) {
+                     size_t workspace_bytes, hipStream_t s, const pq::NormArgs* norm = nullptr) {
   PQ_REQUIRE(count >= 1 && count <= pq::kMaxGroup, PQ_ERR_ARG, "%s: count=%d not in 1..%d", who, count,
              pq::kMaxGroup);
   PQ_REQUIRE(members != nullptr, PQ_ERR_ARG, "%s: null member table", who);
@@ -594,8 +594,9 @@ int w16_linear_group(const char* who, const void* x, int x_dtype, const pq_linea
     gg.mem[i] = {reinterpret_cast<const uint16_t*>(rows), mb.wpack, mb.wmeta, mb.bias, mb.y, static_cast<int>(mb.n)};
   }
   const unsigned rflags = flags | PQ_RQ_MATERIALIZE_FP16;
-  if (split) pq::launch_rotate_split(x, x_dtype, rg, M, K, krot, rflags, s);
-  else pq::launch_rotate_quant_group(x, x_dtype, rg, m, K, krot, rflags, s);
+  // One row per wave, as the W4A8 linear's split rotation.
+  if (split) pq::launch_rotate_split(x, x_dtype, rg, M, K, krot, rflags, s, norm, 1);
+  else pq::launch_rotate_quant_group(x, x_dtype, rg, m, K, krot, rflags, s, norm);
   int st = pq::launch_status("W4A16 linear rotation launch");
   if (st != PQ_OK) return st;
   launch_w16_gemm_group(gg, bias_dtype, y_dtype, M, K, s);
@@ -623,4 +624,16 @@ extern "C" int pq_w4a16_linear_group(const void* x, int x_dtype, const pq_linear
                                      void* workspace, size_t workspace_bytes, void* stream) {
   return w16_linear_group("pq_w4a16_linear_group", x, x_dtype, members, count, bias_dtype, y_dtype, m, k, krot, flags,
                           workspace, workspace_bytes, static_cast<hipStream_t>(stream));
+}
+
+extern "C" int pq_w4a16_linear_group_fused(const void* x, const void* x2, const void* norm_weight, float eps, int mode,
+                                           void* h_out, void* sum_out, int x_dtype, const pq_linear_member* members,
+                                           int count, int bias_dtype, int y_dtype, int64_t m, int64_t k, int krot,
+                                           unsigned flags, void* workspace, size_t workspace_bytes, void* stream) {
+  const char* who = "pq_w4a16_linear_group_fused";
+  pq::NormArgs pro{};
+  const int st = pq::prologue_args(who, x2, norm_weight, eps, mode, h_out, sum_out, x_dtype, m, &pro);
+  if (st != PQ_OK) return st;
+  return w16_linear_group(who, x, x_dtype, members, count, bias_dtype, y_dtype, m, k, krot, flags, workspace,
+                          workspace_bytes, static_cast<hipStream_t>(stream), &pro);
 }

@@ -17,6 +17,9 @@ the ``paroquant`` namespace:
   paroquant::w4a8_linear_group(x, rot_idx[], rot_cs[], scales?[], krot, wpack[], wmeta[], bias?[],
                                input_fp16, materialize_fp16, out_dtype) -> y[]
       (1..4 linears sharing the input x, in two launches for the whole group)
+  paroquant::w4a16_linear_group(x, <rotation and weight lists>, input_fp16, out_dtype, mode=0, x2=None,
+                                norm_weight=None, eps=0, return_h=False, return_sum=False) -> y[] (+ h) (+ x + x2)
+      (the W4A16 group; with a mode behind a decoder layer's elementwise step, folded into its rotation launch)
   paroquant::w4a8_linear_group_rmsnorm(x, residual?, norm_weight, eps, <the group's arguments>,
                                        return_normed, return_sum) -> y[] (+ h) (+ x + residual)
       (the same group behind a decoder layer's RMSNorm of x + residual, still two launches)
@@ -84,7 +87,8 @@ _pq_lib.define("w4a16_prepack(Tensor awq_qweight, Tensor scales, Tensor scaled_z
 _pq_lib.define("w4a16_gemm(Tensor x, Tensor wpack, Tensor wmeta, Tensor? bias, ScalarType out_dtype) -> Tensor")
 _pq_lib.define("w4a16_linear_group(Tensor x, Tensor[] rot_idx, Tensor[] rot_cs, Tensor?[] scales, int krot, "
                "Tensor[] wpack, Tensor[] wmeta, Tensor?[] bias, bool input_fp16, "
-               "ScalarType out_dtype) -> Tensor[]")
+               "ScalarType out_dtype, int mode=0, Tensor? x2=None, Tensor? norm_weight=None, float eps=0.0, "
+               "bool return_h=False, bool return_sum=False) -> Tensor[]")
 _pq_lib.define("w4a16_linear(Tensor x, Tensor rot_idx, Tensor rot_cs, Tensor? scales, int krot, Tensor wpack, "
                "Tensor wmeta, Tensor? bias, bool input_fp16, ScalarType out_dtype) -> Tensor")
 
@@ -664,8 +668,13 @@ def _linear_group_impl(x, rot_idx, rot_cs, scales, krot, wpack, wmeta, bias, inp
     return [y.view(*x.shape[:-1], y.size(1)) for y in outs]
 
 
-def _linear_group_fused_impl(x, x2, norm_weight, eps, mode, rot_idx, rot_cs, scales, krot, wpack, wmeta, bias,
-                             input_fp16, materialize_fp16, out_dtype, return_h, return_sum):
+def _aligned16(t):
+    """t, or a fresh copy of it where a view starts off a 16-byte boundary (the kernels load rows 16 bytes wide)."""
+    return t if t is None or t.data_ptr() % 16 == 0 else t.clone()
+
+
+def _prologue_args(x, x2, norm_weight, mode, return_h, return_sum):
+    """Checks of a fused group's elementwise step; contiguous x, x2 and norm_weight."""
     dev = x.device
     _require(x.dtype in _DT, f"x must be float32/float16/bfloat16, got {x.dtype}")
     _require(mode in (_lib.PQ_PRO_RMSNORM, _lib.PQ_PRO_ADD, _lib.PQ_PRO_SWIGLU), f"unknown prologue mode {mode}")
@@ -687,6 +696,15 @@ def _linear_group_fused_impl(x, x2, norm_weight, eps, mode, rot_idx, rot_cs, sca
     _require(not return_sum or (other is not None and mode != _lib.PQ_PRO_SWIGLU),
              "return_sum needs a residual (RMSNorm with residual, or the add)")
     _require(not return_h or mode != _lib.PQ_PRO_ADD, "the add has no h: use return_sum")
+    return xc, other, w
+
+
+def _linear_group_fused_impl(x, x2, norm_weight, eps, mode, rot_idx, rot_cs, scales, krot, wpack, wmeta, bias,
+                             input_fp16, materialize_fp16, out_dtype, return_h, return_sum):
+    xc, other, w = _prologue_args(x, x2, norm_weight, mode, return_h, return_sum)
+    if mode == _lib.PQ_PRO_SWIGLU:   # (any gate and up run: torch's operations took them at every offset)
+        xc, other = _aligned16(xc), _aligned16(other)
+    dev, k = x.device, xc.size(-1)
     members, outs, keep, bias_dt, m, _ = _group_members(xc, rot_idx, rot_cs, scales, krot, wpack, wmeta, bias,
                                                         out_dtype)
     count = len(outs)
@@ -966,11 +984,19 @@ def _w16_linear_impl(x, rot_idx, rot_cs, scales, krot, wpack, wmeta, bias, input
 _pq_lib.impl("w4a16_linear", _w16_linear_impl, "CUDA")
 
 
-def _w16_linear_group_impl(x, rot_idx, rot_cs, scales, krot, wpack, wmeta, bias, input_fp16, out_dtype):
-    """paroquant::w4a16_linear for linears that read the same x, in one rotation launch and (m <= 16) one GEMM."""
+def _w16_linear_group_impl(x, rot_idx, rot_cs, scales, krot, wpack, wmeta, bias, input_fp16, out_dtype, mode=0,
+                           x2=None, norm_weight=None, eps=0.0, return_h=False, return_sum=False):
+    """paroquant::w4a16_linear for linears that read the same x, in one rotation launch and (m <= 16) one GEMM;
+    with a mode (PQ_PRO_*) behind that elementwise step, which runs inside the rotation launch."""
     dev = x.device
     _require(x.dtype in _DT, f"x must be float32/float16/bfloat16, got {x.dtype}")
-    xc = x.contiguous()
+    _require(mode != 0 or not (x2 is not None or norm_weight is not None or return_h or return_sum),
+             "x2, norm_weight, return_h and return_sum need a mode")
+    if mode:
+        xc, other, w = _prologue_args(x, x2, norm_weight, mode, return_h, return_sum)
+        xc, other = _aligned16(xc), _aligned16(other)
+    else:
+        xc = x.contiguous()
     members, outs, keep, bias_dt, m, k = _group_members(xc, rot_idx, rot_cs, scales, krot, wpack, wmeta, bias,
                                                         out_dtype)
     count = len(outs)
@@ -978,20 +1004,32 @@ def _w16_linear_group_impl(x, rot_idx, rot_cs, scales, krot, wpack, wmeta, bias,
     need = int(lib.pq_w4a16_linear_group_workspace_size(m, k, count))
     scratch = torch.empty(need, dtype=torch.uint8, device=dev) if need > 0 else None
     flags = _lib.PQ_RQ_INPUT_FP16 if input_fp16 else 0
+    h = torch.empty_like(xc) if return_h else None
+    sm = torch.empty_like(xc) if return_sum else None
+    rest = (_DT[x.dtype], members, count, bias_dt, _DT[out_dtype], m, k, krot, flags,
+            scratch.data_ptr() if scratch is not None else None, scratch.numel() if scratch is not None else 0)
     with _DeviceGuard(dev):
-        st = lib.pq_w4a16_linear_group(xc.data_ptr(), _DT[x.dtype], members, count, bias_dt, _DT[out_dtype], m, k,
-                                       krot, flags, scratch.data_ptr() if scratch is not None else None,
-                                       scratch.numel() if scratch is not None else 0, _stream(dev))
+        if mode:
+            st = lib.pq_w4a16_linear_group_fused(
+                xc.data_ptr(), other.data_ptr() if other is not None else None,
+                w.data_ptr() if w is not None else None, float(eps), int(mode),
+                h.data_ptr() if h is not None else None, sm.data_ptr() if sm is not None else None, *rest,
+                _stream(dev))
+        else:
+            st = lib.pq_w4a16_linear_group(xc.data_ptr(), *rest, _stream(dev))
     _lib.check(st, "paroquant::w4a16_linear_group")
-    return [y.view(*x.shape[:-1], y.size(1)) for y in outs]
+    res_out = [y.view(*x.shape[:-1], y.size(1)) for y in outs]
+    return res_out + [t.view(x.shape) for t in (h, sm) if t is not None]
 
 
 _pq_lib.impl("w4a16_linear_group", _w16_linear_group_impl, "CUDA")
 
 
 @torch.library.register_fake("paroquant::w4a16_linear_group")
-def _w16_linear_group_fake(x, rot_idx, rot_cs, scales, krot, wpack, wmeta, bias, input_fp16, out_dtype):
-    return [x.new_empty((*x.shape[:-1], w.size(0) * 16), dtype=out_dtype) for w in wpack]
+def _w16_linear_group_fake(x, rot_idx, rot_cs, scales, krot, wpack, wmeta, bias, input_fp16, out_dtype, mode=0,
+                           x2=None, norm_weight=None, eps=0.0, return_h=False, return_sum=False):
+    outs = [x.new_empty((*x.shape[:-1], w.size(0) * 16), dtype=out_dtype) for w in wpack]
+    return outs + [x.new_empty(x.shape) for want in (return_h, return_sum) if want]
 
 
 @torch.library.register_fake("paroquant::w4a16_linear")

@@ -41,6 +41,8 @@
  *                        (rotation_linear.py:136-139)
  *   pq_w4a16_linear_group  the same for linears sharing their input
  *                        (no counterpart)
+ *   pq_w4a16_linear_group_fused  the same behind a decoder layer's
+ *                        elementwise step (no counterpart)
  */
 #ifndef PAROQUANT_HIP_H
 #define PAROQUANT_HIP_H
@@ -366,6 +368,14 @@ size_t pq_w4a16_linear_group_workspace_size(int64_t m, int64_t k, int count);
 int pq_w4a16_linear_group(const void* x, int x_dtype, const pq_linear_member* members, int count,
                           int bias_dtype, int y_dtype, int64_t m, int64_t k, int krot, unsigned flags,
                           void* workspace, size_t workspace_bytes, void* stream);
+
+/* pq_w4a16_linear_group behind a decoder layer's elementwise step: x2,
+ * norm_weight, eps, mode, h_out and sum_out as for
+ * pq_w4a8_linear_group_fused, the step folded into the rotation launch. */
+int pq_w4a16_linear_group_fused(const void* x, const void* x2, const void* norm_weight, float eps, int mode,
+                                void* h_out, void* sum_out, int x_dtype, const pq_linear_member* members, int count,
+                                int bias_dtype, int y_dtype, int64_t m, int64_t k, int krot, unsigned flags,
+                                void* workspace, size_t workspace_bytes, void* stream);
 
 /* pq_w4a8_linear_group behind a decoder layer's elementwise step, chosen by
  * mode (PQ_PRO_*), in the same two launches; the members read
