@@ -16,6 +16,7 @@
 #include <algorithm>
 #include <type_traits>
 
+#include "pq_chain.h"
 #include "pq_device.h"
 #include "pq_internal.h"
 
@@ -421,10 +422,39 @@ void launch_rotate(const void* x, void* y, uint8_t* sc, const int16_t* idx, cons
                                                                             krot);
 }
 
+// The register chain (pq_chain.h) from 4 M elements on: below, a workgroup's
+// chain serves too few rows to pay for being derived (fp16, 8 layers, tile
+// form -> chain in us: 512 x 4096 9.6 -> 10.0, 1024 x 4096 15.6 -> 12.9, 2100 x
+// 4096 27.3 -> 20.1, 1024 x 12288 37.4 -> 25.7; 16 layers 1024 x 4096 24.1 ->
+// 18.7; float32, 8 layers, 8192 x 4096 102 -> 58).
+constexpr int64_t kChainElems = 1 << 22;
+
+template <int DT, bool MX>
+void launch_chain(const void* x, void* y, uint8_t* sc, const int16_t* idx, const void* theta, const void* scales,
+                  int64_t rows, int h, int krot, int group, hipStream_t stream) {
+  // Slices of the rows for the two workgroups a CU holds, in whole steps of 32 rows.
+  const int64_t chunks = (h + 127) / 128;
+  const int64_t want = std::max<int64_t>(1, 512 / chunks);
+  const int64_t slice = ((rows + want - 1) / want + 31) / 32 * 32;
+  const dim3 grid(static_cast<unsigned>((rows + slice - 1) / slice), static_cast<unsigned>(chunks));
+#define PQ_CHAIN(K_)                                                                                                 \
+  case K_:                                                                                                           \
+    pqchain::rotate_chain<DT, K_, MX><<<grid, pqchain::kWaves * 64, 0, stream>>>(x, y, sc, idx, theta, scales, rows, \
+                                                                                 h, group, slice);                   \
+    break;
+  switch (krot) { PQ_CHAIN(1) PQ_CHAIN(2) PQ_CHAIN(4) PQ_CHAIN(8) PQ_CHAIN(16) }
+#undef PQ_CHAIN
+}
+
 // sc == nullptr: rotated values into y; else MXFP4 codes into y, scales into sc.
 template <int DT>
 void launch_rotate_dt(const void* x, void* y, uint8_t* sc, const int16_t* idx, const void* theta,
                       const void* scales, int64_t rows, int h, int krot, int group, hipStream_t stream) {
+  if (rows * h >= kChainElems) {
+    if (sc != nullptr) launch_chain<DT, true>(x, y, sc, idx, theta, scales, rows, h, krot, group, stream);
+    else launch_chain<DT, false>(x, y, sc, idx, theta, scales, rows, h, krot, group, stream);
+    return;
+  }
   if (group == 128) {
     if (scales) launch_rotate<DT, 128, true>(x, y, sc, idx, theta, scales, rows, h, krot, stream);
     else launch_rotate<DT, 128, false>(x, y, sc, idx, theta, scales, rows, h, krot, stream);
