@@ -98,7 +98,8 @@ _pq_lib.define("w4a16_linear(Tensor x, Tensor rot_idx, Tensor rot_cs, Tensor? sc
 # ---------------------------------------------------------------------------
 
 def _stream(dev: torch.device) -> int:
-    return torch.cuda.current_stream(dev).cuda_stream
+    # the current stream's handle without the torch.cuda.Stream object around it
+    return torch._C._cuda_getCurrentRawStream(dev.index)
 
 
 class _DeviceGuard:
@@ -111,7 +112,7 @@ class _DeviceGuard:
         self.prev = None
 
     def __enter__(self):
-        cur = torch.cuda.current_device()
+        cur = torch._C._cuda_getDevice()
         if self.dev.index is not None and self.dev.index != cur:
             self.prev = cur
             torch.cuda.set_device(self.dev)
@@ -123,20 +124,17 @@ class _DeviceGuard:
         return False
 
 
-def _require(cond: bool, msg: str) -> None:
-    if not cond:
-        raise RuntimeError(msg)
-
-
 def _same_device(name: str, t: torch.Tensor, dev: torch.device) -> None:
-    _require(t.device == dev, f"{name}: expected a tensor on {dev}, got {t.device}")
+    if not (t.device == dev):
+        raise RuntimeError(f"{name}: expected a tensor on {dev}, got {t.device}")
 
 
 def gemm_dims(wpack: torch.Tensor) -> tuple[int, int]:
     """(out_features, in_features) of a prepacked weight [N/16, K/128, 64, 16]."""
-    _require(wpack.dim() == 4 and wpack.size(2) == 64 and wpack.size(3) == 16 and wpack.dtype == torch.uint8,
-             "wpack must be uint8 [N/16, K/128, 64, 16]")
-    return wpack.size(0) * 16, wpack.size(1) * 128
+    sp = wpack.shape
+    if not (len(sp) == 4 and sp[2] == 64 and sp[3] == 16 and wpack.dtype == torch.uint8):
+        raise RuntimeError("wpack must be uint8 [N/16, K/128, 64, 16]")
+    return sp[0] * 16, sp[1] * 128
 
 
 def workspace_bytes(m: int, n: int, k: int) -> int:
@@ -154,20 +152,29 @@ def linear_workspace_bytes(m: int, n: int, k: int, krot: int) -> int:
 
 def _rotate_args(x, idx_ij, theta, scales):
     """Checks of rotation::rotate's arguments; contiguous copies and the sizes."""
-    _require(x.dtype in _DT, f"rotate only supports Float, Half, and BFloat16, but got {x.dtype}")
-    _require(idx_ij.dtype == torch.int16, f"idx_ij must be int16, got {idx_ij.dtype}")
-    _require(theta.dtype == x.dtype, f"theta must have x's dtype {x.dtype}, got {theta.dtype}")
-    _require(x.dim() >= 1 and x.size(-1) > 0, "x must have a non-empty last dimension")
+    if not (x.dtype in _DT):
+        raise RuntimeError(f"rotate only supports Float, Half, and BFloat16, but got {x.dtype}")
+    if not (idx_ij.dtype == torch.int16):
+        raise RuntimeError(f"idx_ij must be int16, got {idx_ij.dtype}")
+    if not (theta.dtype == x.dtype):
+        raise RuntimeError(f"theta must have x's dtype {x.dtype}, got {theta.dtype}")
+    if not (x.dim() >= 1 and x.size(-1) > 0):
+        raise RuntimeError("x must have a non-empty last dimension")
     h = x.size(-1)
-    _require(idx_ij.dim() == 2 and theta.dim() == 2, "idx_ij and theta must be 2-D [KROT, H] / [KROT, H/2]")
+    if not (idx_ij.dim() == 2 and theta.dim() == 2):
+        raise RuntimeError("idx_ij and theta must be 2-D [KROT, H] / [KROT, H/2]")
     krot = theta.size(0)
-    _require(krot == idx_ij.size(0), "theta.size(0) must equal idx_ij.size(0)")
-    _require(idx_ij.size(1) == h and theta.size(1) * 2 == h,
-             f"idx_ij must be [KROT, {h}] and theta [KROT, {h // 2}], got {tuple(idx_ij.shape)} / {tuple(theta.shape)}")
+    if not (krot == idx_ij.size(0)):
+        raise RuntimeError("theta.size(0) must equal idx_ij.size(0)")
+    if not (idx_ij.size(1) == h and theta.size(1) * 2 == h):
+        raise RuntimeError(f"idx_ij must be [KROT, {h}] and theta [KROT, {h // 2}], got {tuple(idx_ij.shape)} / "
+                           f"{tuple(theta.shape)}")
     has_scale = scales is not None and scales.numel() > 0
     if has_scale:
-        _require(scales.dtype == x.dtype, f"scales must have x's dtype {x.dtype}, got {scales.dtype}")
-        _require(scales.numel() == h, f"scales must hold {h} values, got {scales.numel()}")
+        if not (scales.dtype == x.dtype):
+            raise RuntimeError(f"scales must have x's dtype {x.dtype}, got {scales.dtype}")
+        if not (scales.numel() == h):
+            raise RuntimeError(f"scales must hold {h} values, got {scales.numel()}")
     dev = x.device
     for nm, t in (("idx_ij", idx_ij), ("theta", theta)) + ((("scales", scales),) if has_scale else ()):
         _same_device(nm, t, dev)
@@ -276,7 +283,8 @@ def _rotate_impl(x, idx_ij, theta, scales, group_size):
 
 def _rotate_mxfp4_impl(x, idx_ij, theta, scales, group_size):
     xc, idc, thc, scc, rows, h, krot = _rotate_args(x, idx_ij, theta, scales)
-    _require(h % 32 == 0, f"MXFP4 blocks are 32 channels: h={h}")
+    if not (h % 32 == 0):
+        raise RuntimeError(f"MXFP4 blocks are 32 channels: h={h}")
     dev = x.device
     q = torch.empty((*x.shape[:-1], h // 2), dtype=torch.uint8, device=dev)
     sc = torch.empty((*x.shape[:-1], h // 32), dtype=torch.uint8, device=dev)
@@ -314,8 +322,9 @@ def _rotate_mxfp4_fake(x, idx_ij, theta, scales, group_size):
 
 def _rotate_backward_impl(grad_y, x, idx_ij, theta, scales, group_size):
     xc, idc, thc, scc, rows, h, krot = _rotate_args(x, idx_ij, theta, scales)
-    _require(grad_y.shape == x.shape and grad_y.dtype == x.dtype,
-             f"grad_y must match x ({tuple(x.shape)}, {x.dtype}), got {tuple(grad_y.shape)}, {grad_y.dtype}")
+    if not (grad_y.shape == x.shape and grad_y.dtype == x.dtype):
+        raise RuntimeError(f"grad_y must match x ({tuple(x.shape)}, {x.dtype}), got {tuple(grad_y.shape)}, "
+                           f"{grad_y.dtype}")
     dev = x.device
     _same_device("grad_y", grad_y, dev)
     gyc = grad_y.contiguous()
@@ -361,7 +370,8 @@ def pack_rotation(pairs: torch.Tensor, cos_sin: torch.Tensor) -> tuple[torch.Ten
     p = pairs.detach().to("cpu", torch.int16).contiguous()
     cs = cos_sin.detach().to("cpu", torch.float32).contiguous()
     krot, h = p.shape
-    _require(tuple(cs.shape) == (krot, h // 2, 2), f"cos_sin must be [{krot}, {h // 2}, 2]")
+    if not (cs.shape == (krot, h // 2, 2)):
+        raise RuntimeError(f"cos_sin must be [{krot}, {h // 2}, 2]")
     sij, scs = packed_rotation_shapes(h, krot)
     rot_idx = torch.empty(sij, dtype=torch.int32)
     rot_cs = torch.empty(scs, dtype=torch.float32)
@@ -374,17 +384,20 @@ def pack_rotation(pairs: torch.Tensor, cos_sin: torch.Tensor) -> tuple[torch.Ten
 
 def _check_rot_params(x, rot_idx, rot_cs, scales, krot):
     h = x.size(-1)
-    _require(x.dtype in _DT, f"x must be float32/float16/bfloat16, got {x.dtype}")
-    _require(h % 128 == 0 and 0 < h <= 16384, f"in_features={h} must be a multiple of 128 and <= 16384")
-    _require(1 <= krot <= 16, f"KROT={krot} must be in 1..16")
+    if not (x.dtype in _DT):
+        raise RuntimeError(f"x must be float32/float16/bfloat16, got {x.dtype}")
+    if not (h % 128 == 0 and 0 < h <= 16384):
+        raise RuntimeError(f"in_features={h} must be a multiple of 128 and <= 16384")
+    if not (1 <= krot <= 16):
+        raise RuntimeError(f"KROT={krot} must be in 1..16")
     sij, scs = packed_rotation_shapes(h, krot)
-    _require(rot_idx.dtype in (torch.int32, torch.uint32) and tuple(rot_idx.shape) == sij,
-             f"rot_idx must be int32 {sij}, got {rot_idx.dtype} {tuple(rot_idx.shape)}")
-    _require(rot_cs.dtype == torch.float32 and tuple(rot_cs.shape) == scs,
-             f"rot_cs must be float32 {scs}, got {rot_cs.dtype} {tuple(rot_cs.shape)}")
+    if not (rot_idx.dtype in (torch.int32, torch.uint32) and rot_idx.shape == sij):
+        raise RuntimeError(f"rot_idx must be int32 {sij}, got {rot_idx.dtype} {tuple(rot_idx.shape)}")
+    if not (rot_cs.dtype == torch.float32 and rot_cs.shape == scs):
+        raise RuntimeError(f"rot_cs must be float32 {scs}, got {rot_cs.dtype} {tuple(rot_cs.shape)}")
     if scales is not None:
-        _require(scales.dtype == torch.float32 and scales.numel() == h,
-                 f"scales must be float32 with {h} values, got {scales.dtype} {scales.numel()}")
+        if not (scales.dtype == torch.float32 and scales.numel() == h):
+            raise RuntimeError(f"scales must be float32 with {h} values, got {scales.dtype} {scales.numel()}")
     dev = x.device
     _same_device("rot_idx", rot_idx, dev)
     _same_device("rot_cs", rot_cs, dev)
@@ -442,9 +455,11 @@ def _rotate_quant_rot_fake(x, rot_idx, rot_cs, scales, krot, input_fp16, materia
 
 
 def _quant_impl(x):
-    _require(x.dtype in _DT, f"x must be float32/float16/bfloat16, got {x.dtype}")
+    if not (x.dtype in _DT):
+        raise RuntimeError(f"x must be float32/float16/bfloat16, got {x.dtype}")
     h = x.size(-1)
-    _require(h % 8 == 0 and h > 0, f"last dimension {h} must be a positive multiple of 8")
+    if not (h % 8 == 0 and h > 0):
+        raise RuntimeError(f"last dimension {h} must be a positive multiple of 8")
     dev = x.device
     xc = x.contiguous()
     rows = xc.numel() // h
@@ -473,19 +488,22 @@ def _quant_fake(x):
 
 def _check_weights(wpack, wmeta, dev):
     n, k = gemm_dims(wpack)
-    _require(wmeta.dtype in (torch.int32, torch.uint32) and tuple(wmeta.shape) == (n // 16, k // 128, 16),
-             f"wmeta must be int32 [{n // 16}, {k // 128}, 16], got {wmeta.dtype} {tuple(wmeta.shape)}")
-    _require(wpack.is_contiguous() and wmeta.is_contiguous(), "wpack/wmeta must be contiguous")
+    if not (wmeta.dtype in (torch.int32, torch.uint32) and wmeta.shape == (n // 16, k // 128, 16)):
+        raise RuntimeError(f"wmeta must be int32 [{n // 16}, {k // 128}, 16], got {wmeta.dtype} {tuple(wmeta.shape)}")
+    if not (wpack.is_contiguous() and wmeta.is_contiguous()):
+        raise RuntimeError("wpack/wmeta must be contiguous")
     _same_device("wpack", wpack, dev)
     _same_device("wmeta", wmeta, dev)
     return n, k
 
 
 def _gemm_launch(xq, xs, wpack, wmeta, bias, out_dtype, m, n, k, dev):
-    _require(out_dtype in _DT, f"out_dtype must be float32/float16/bfloat16, got {out_dtype}")
+    if not (out_dtype in _DT):
+        raise RuntimeError(f"out_dtype must be float32/float16/bfloat16, got {out_dtype}")
     y = torch.empty((m, n), dtype=out_dtype, device=dev)
     if bias is not None:
-        _require(bias.dtype in _DT and bias.numel() == n, f"bias must hold {n} float values")
+        if not (bias.dtype in _DT and bias.numel() == n):
+            raise RuntimeError(f"bias must hold {n} float values")
         _same_device("bias", bias, dev)
         bias = bias.contiguous()
     need = workspace_bytes(m, n, k)
@@ -506,10 +524,11 @@ def _gemm_launch(xq, xs, wpack, wmeta, bias, out_dtype, m, n, k, dev):
 def _gemm_impl(xq, xscale, wpack, wmeta, bias, out_dtype):
     dev = xq.device
     n, k = _check_weights(wpack, wmeta, dev)
-    _require(xq.dtype == torch.int8 and xq.dim() == 2 and xq.size(1) == k,
-             f"xq must be int8 [M, {k}], got {xq.dtype} {tuple(xq.shape)}")
+    if not (xq.dtype == torch.int8 and xq.dim() == 2 and xq.size(1) == k):
+        raise RuntimeError(f"xq must be int8 [M, {k}], got {xq.dtype} {tuple(xq.shape)}")
     m = xq.size(0)
-    _require(xscale.dtype == torch.float32 and xscale.numel() == m, f"xscale must be float32 [{m}]")
+    if not (xscale.dtype == torch.float32 and xscale.numel() == m):
+        raise RuntimeError(f"xscale must be float32 [{m}]")
     _same_device("xscale", xscale, dev)
     return _gemm_launch(xq.contiguous(), xscale.contiguous(), wpack, wmeta, bias, out_dtype, m, n, k, dev)
 
@@ -525,7 +544,8 @@ def _gemm_fake(xq, xscale, wpack, wmeta, bias, out_dtype):
 def _partials_impl(xq, wpack, wmeta):
     dev = xq.device
     n, k = _check_weights(wpack, wmeta, dev)
-    _require(xq.dtype == torch.int8 and xq.dim() == 2 and xq.size(1) == k, f"xq must be int8 [M, {k}]")
+    if not (xq.dtype == torch.int8 and xq.dim() == 2 and xq.size(1) == k):
+        raise RuntimeError(f"xq must be int8 [M, {k}]")
     m = xq.size(0)
     out = torch.empty((m, k // 128, n), dtype=torch.int32, device=dev)
     xc = xq.contiguous()
@@ -547,14 +567,17 @@ def _partials_fake(xq, wpack, wmeta):
 
 def _prepack_impl(awq_qweight, awq_scales, awq_qzeros):
     dev = awq_qweight.device
-    _require(awq_qweight.dtype == torch.int32 and awq_qweight.dim() == 2, "awq_qweight must be int32 [K, N/8]")
+    if not (awq_qweight.dtype == torch.int32 and awq_qweight.dim() == 2):
+        raise RuntimeError("awq_qweight must be int32 [K, N/8]")
     k, n = awq_qweight.size(0), awq_qweight.size(1) * 8
-    _require(k % 128 == 0 and n % 16 == 0, f"K={k} must be a multiple of 128 and N={n} of 16")
+    if not (k % 128 == 0 and n % 16 == 0):
+        raise RuntimeError(f"K={k} must be a multiple of 128 and N={n} of 16")
     g = k // 128
-    _require(awq_scales.dtype == torch.float16 and tuple(awq_scales.shape) == (g, n),
-             f"awq_scales must be float16 [{g}, {n}], got {awq_scales.dtype} {tuple(awq_scales.shape)}")
-    _require(awq_qzeros.dtype == torch.int32 and tuple(awq_qzeros.shape) == (g, n // 8),
-             f"awq_qzeros must be int32 [{g}, {n // 8}], got {awq_qzeros.dtype} {tuple(awq_qzeros.shape)}")
+    if not (awq_scales.dtype == torch.float16 and awq_scales.shape == (g, n)):
+        raise RuntimeError(f"awq_scales must be float16 [{g}, {n}], got {awq_scales.dtype} {tuple(awq_scales.shape)}")
+    if not (awq_qzeros.dtype == torch.int32 and awq_qzeros.shape == (g, n // 8)):
+        raise RuntimeError(f"awq_qzeros must be int32 [{g}, {n // 8}], got {awq_qzeros.dtype} "
+                           f"{tuple(awq_qzeros.shape)}")
     _same_device("awq_scales", awq_scales, dev)
     _same_device("awq_qzeros", awq_qzeros, dev)
     qw, sc, qz = awq_qweight.contiguous(), awq_scales.contiguous(), awq_qzeros.contiguous()
@@ -581,14 +604,17 @@ def _prepack_fake(awq_qweight, awq_scales, awq_qzeros):
 def _linear_impl(x, rot_idx, rot_cs, scales, krot, wpack, wmeta, bias, input_fp16, materialize_fp16, out_dtype):
     dev = x.device
     n, k = _check_weights(wpack, wmeta, dev)
-    _require(x.size(-1) == k, f"x has {x.size(-1)} features, the weights expect {k}")
+    if not (x.size(-1) == k):
+        raise RuntimeError(f"x has {x.size(-1)} features, the weights expect {k}")
     _check_rot_params(x, rot_idx, rot_cs, scales, krot)
-    _require(out_dtype in _DT, f"out_dtype must be float32/float16/bfloat16, got {out_dtype}")
+    if not (out_dtype in _DT):
+        raise RuntimeError(f"out_dtype must be float32/float16/bfloat16, got {out_dtype}")
     xc = x.contiguous()
     m = xc.numel() // k
     y = torch.empty((m, n), dtype=out_dtype, device=dev)
     if bias is not None:
-        _require(bias.dtype in _DT and bias.numel() == n, f"bias must hold {n} float values")
+        if not (bias.dtype in _DT and bias.numel() == n):
+            raise RuntimeError(f"bias must hold {n} float values")
         _same_device("bias", bias, dev)
         bias = bias.contiguous()
     lib = _lib.load()
@@ -606,7 +632,7 @@ def _linear_impl(x, rot_idx, rot_cs, scales, krot, wpack, wmeta, bias, input_fp1
                                 scratch.numel() if scratch is not None else 0,
                                 _stream(dev))
     _lib.check(st, "paroquant::w4a8_linear")
-    return y.view(*x.shape[:-1], n)
+    return y if x.dim() == 2 else y.view(*x.shape[:-1], n)
 
 
 _pq_lib.impl("w4a8_linear", _linear_impl, "CUDA")
@@ -616,26 +642,31 @@ def _group_members(x, rot_idx, rot_cs, scales, krot, wpack, wmeta, bias, out_dty
     """The pq_linear_member table of a group over x [.., k], the outputs it writes, and what must stay alive."""
     dev = x.device
     count = len(wpack)
-    _require(1 <= count <= _lib.MAX_GROUP, f"a group holds 1..{_lib.MAX_GROUP} linears, got {count}")
-    _require(len(rot_idx) == len(rot_cs) == len(scales) == len(wmeta) == len(bias) == count,
-             "every per-member list must have one entry per linear")
-    _require(out_dtype in _DT, f"out_dtype must be float32/float16/bfloat16, got {out_dtype}")
+    if not (1 <= count <= _lib.MAX_GROUP):
+        raise RuntimeError(f"a group holds 1..{_lib.MAX_GROUP} linears, got {count}")
+    if not (len(rot_idx) == len(rot_cs) == len(scales) == len(wmeta) == len(bias) == count):
+        raise RuntimeError("every per-member list must have one entry per linear")
+    if not (out_dtype in _DT):
+        raise RuntimeError(f"out_dtype must be float32/float16/bfloat16, got {out_dtype}")
     k = x.size(-1)
     m = x.numel() // k
     members = (_lib.LinearMember * count)()
     keep, outs, bias_dt = [], [], 0
     for i in range(count):
         n, kw = _check_weights(wpack[i], wmeta[i], dev)
-        _require(kw == k, f"member {i}: the weights expect {kw} features, x has {k}")
+        if not (kw == k):
+            raise RuntimeError(f"member {i}: the weights expect {kw} features, x has {k}")
         _check_rot_params(x, rot_idx[i], rot_cs[i], scales[i], krot)
         idx, cs = rot_idx[i].contiguous(), rot_cs[i].contiguous()
         sc = scales[i].contiguous() if scales[i] is not None else None
         b = bias[i]
         if b is not None:
-            _require(b.dtype in _DT and b.numel() == n, f"member {i}: bias must hold {n} float values")
+            if not (b.dtype in _DT and b.numel() == n):
+                raise RuntimeError(f"member {i}: bias must hold {n} float values")
             _same_device("bias", b, dev)
             b = b.contiguous()
-            _require(bias_dt in (0, _DT[b.dtype]), "all biases of a group must share one dtype")
+            if not (bias_dt in (0, _DT[b.dtype])):
+                raise RuntimeError("all biases of a group must share one dtype")
             bias_dt = _DT[b.dtype]
         y = torch.empty((m, n), dtype=out_dtype, device=dev)
         keep += [idx, cs, sc, b]
@@ -679,26 +710,31 @@ def _aligned16(t):
 def _prologue_args(x, x2, norm_weight, mode, return_h, return_sum):
     """Checks of a fused group's elementwise step; contiguous x, x2 and norm_weight."""
     dev = x.device
-    _require(x.dtype in _DT, f"x must be float32/float16/bfloat16, got {x.dtype}")
-    _require(mode in (_lib.PQ_PRO_RMSNORM, _lib.PQ_PRO_ADD, _lib.PQ_PRO_SWIGLU), f"unknown prologue mode {mode}")
+    if not (x.dtype in _DT):
+        raise RuntimeError(f"x must be float32/float16/bfloat16, got {x.dtype}")
+    if not (mode in (_lib.PQ_PRO_RMSNORM, _lib.PQ_PRO_ADD, _lib.PQ_PRO_SWIGLU)):
+        raise RuntimeError(f"unknown prologue mode {mode}")
     xc = x.contiguous()
     k = xc.size(-1)
     w = None
     if mode == _lib.PQ_PRO_RMSNORM:
-        _require(norm_weight is not None and norm_weight.dtype == x.dtype and norm_weight.numel() == k,
-                 f"norm_weight must hold {k} values of x's dtype {x.dtype}")
+        if not (norm_weight is not None and norm_weight.dtype == x.dtype and norm_weight.numel() == k):
+            raise RuntimeError(f"norm_weight must hold {k} values of x's dtype {x.dtype}")
         _same_device("norm_weight", norm_weight, dev)
         w = norm_weight.contiguous()
     else:
-        _require(x2 is not None, "the add and the SwiGLU need x2 (residual / up)")
+        if not (x2 is not None):
+            raise RuntimeError("the add and the SwiGLU need x2 (residual / up)")
     other = None
     if x2 is not None:
-        _require(x2.shape == x.shape and x2.dtype == x.dtype, "x2 (residual / up) must match x's shape and dtype")
+        if not (x2.shape == x.shape and x2.dtype == x.dtype):
+            raise RuntimeError("x2 (residual / up) must match x's shape and dtype")
         _same_device("x2", x2, dev)
         other = x2.contiguous()
-    _require(not return_sum or (other is not None and mode != _lib.PQ_PRO_SWIGLU),
-             "return_sum needs a residual (RMSNorm with residual, or the add)")
-    _require(not return_h or mode != _lib.PQ_PRO_ADD, "the add has no h: use return_sum")
+    if not (not return_sum or (other is not None and mode != _lib.PQ_PRO_SWIGLU)):
+        raise RuntimeError("return_sum needs a residual (RMSNorm with residual, or the add)")
+    if not (not return_h or mode != _lib.PQ_PRO_ADD):
+        raise RuntimeError("the add has no h: use return_sum")
     return xc, other, w
 
 
@@ -843,7 +879,8 @@ def w4a8_linear_group_intermediates(x, rot_idx, rot_cs, scales, krot, wpack, wme
     (codes int8 [count, m, k], xscale float32 [count, m], [partials int32 [m, k/128, n_i] per member],
     h or None, s or None)."""
     dev = x.device
-    _require(x.dtype in _DT, f"x must be float32/float16/bfloat16, got {x.dtype}")
+    if not (x.dtype in _DT):
+        raise RuntimeError(f"x must be float32/float16/bfloat16, got {x.dtype}")
     xc = x.contiguous()
     k = xc.size(-1)
     nb = [None] * len(wpack)
@@ -889,20 +926,23 @@ def _linear_fake(x, rot_idx, rot_cs, scales, krot, wpack, wmeta, bias, input_fp1
 def _w16_bias(bias, n, dev):
     if bias is None:
         return None
-    _require(bias.dtype in _DT and bias.numel() == n, f"bias must hold {n} float values")
+    if not (bias.dtype in _DT and bias.numel() == n):
+        raise RuntimeError(f"bias must hold {n} float values")
     _same_device("bias", bias, dev)
     return bias.contiguous()
 
 
 def _w16_prepack_impl(awq_qweight, scales, scaled_zeros):
     dev = awq_qweight.device
-    _require(awq_qweight.dtype == torch.int32 and awq_qweight.dim() == 2, "awq_qweight must be int32 [K, N/8]")
+    if not (awq_qweight.dtype == torch.int32 and awq_qweight.dim() == 2):
+        raise RuntimeError("awq_qweight must be int32 [K, N/8]")
     k, n = awq_qweight.size(0), awq_qweight.size(1) * 8
-    _require(k % 128 == 0 and n % 16 == 0, f"K={k} must be a multiple of 128 and N={n} of 16")
+    if not (k % 128 == 0 and n % 16 == 0):
+        raise RuntimeError(f"K={k} must be a multiple of 128 and N={n} of 16")
     g = k // 128
     for name, t in (("scales", scales), ("scaled_zeros", scaled_zeros)):
-        _require(t.dtype == torch.float16 and tuple(t.shape) == (g, n),
-                 f"{name} must be float16 [{g}, {n}], got {t.dtype} {tuple(t.shape)}")
+        if not (t.dtype == torch.float16 and t.shape == (g, n)):
+            raise RuntimeError(f"{name} must be float16 [{g}, {n}], got {t.dtype} {tuple(t.shape)}")
         _same_device(name, t, dev)
     qw, sc, sz = awq_qweight.contiguous(), scales.contiguous(), scaled_zeros.contiguous()
     wpack = torch.empty((n // 16, g, 64, 16), dtype=torch.uint8, device=dev)
@@ -928,9 +968,12 @@ def _w16_prepack_fake(awq_qweight, scales, scaled_zeros):
 def _w16_gemm_impl(x, wpack, wmeta, bias, out_dtype):
     dev = x.device
     n, k = _check_weights(wpack, wmeta, dev)
-    _require(x.dtype == torch.float16, f"x must be float16 (the W4A16 kernels take fp16 activations), got {x.dtype}")
-    _require(x.size(-1) == k, f"x has {x.size(-1)} features, the weights expect {k}")
-    _require(out_dtype in _DT, f"out_dtype must be float32/float16/bfloat16, got {out_dtype}")
+    if not (x.dtype == torch.float16):
+        raise RuntimeError(f"x must be float16 (the W4A16 kernels take fp16 activations), got {x.dtype}")
+    if not (x.size(-1) == k):
+        raise RuntimeError(f"x has {x.size(-1)} features, the weights expect {k}")
+    if not (out_dtype in _DT):
+        raise RuntimeError(f"out_dtype must be float32/float16/bfloat16, got {out_dtype}")
     xc = x.contiguous()
     m = xc.numel() // k
     y = torch.empty((m, n), dtype=out_dtype, device=dev)
@@ -960,9 +1003,11 @@ def w4a16_linear_workspace_bytes(m: int, k: int) -> int:
 def _w16_linear_impl(x, rot_idx, rot_cs, scales, krot, wpack, wmeta, bias, input_fp16, out_dtype):
     dev = x.device
     n, k = _check_weights(wpack, wmeta, dev)
-    _require(x.size(-1) == k, f"x has {x.size(-1)} features, the weights expect {k}")
+    if not (x.size(-1) == k):
+        raise RuntimeError(f"x has {x.size(-1)} features, the weights expect {k}")
     _check_rot_params(x, rot_idx, rot_cs, scales, krot)
-    _require(out_dtype in _DT, f"out_dtype must be float32/float16/bfloat16, got {out_dtype}")
+    if not (out_dtype in _DT):
+        raise RuntimeError(f"out_dtype must be float32/float16/bfloat16, got {out_dtype}")
     xc = x.contiguous()
     m = xc.numel() // k
     y = torch.empty((m, n), dtype=out_dtype, device=dev)
@@ -992,9 +1037,10 @@ def _w16_linear_group_impl(x, rot_idx, rot_cs, scales, krot, wpack, wmeta, bias,
     """paroquant::w4a16_linear for linears that read the same x, in one rotation launch and (m <= 16) one GEMM;
     with a mode (PQ_PRO_*) behind that elementwise step, which runs inside the rotation launch."""
     dev = x.device
-    _require(x.dtype in _DT, f"x must be float32/float16/bfloat16, got {x.dtype}")
-    _require(mode != 0 or not (x2 is not None or norm_weight is not None or return_h or return_sum),
-             "x2, norm_weight, return_h and return_sum need a mode")
+    if not (x.dtype in _DT):
+        raise RuntimeError(f"x must be float32/float16/bfloat16, got {x.dtype}")
+    if not (mode != 0 or not (x2 is not None or norm_weight is not None or return_h or return_sum)):
+        raise RuntimeError("x2, norm_weight, return_h and return_sum need a mode")
     if mode:
         xc, other, w = _prologue_args(x, x2, norm_weight, mode, return_h, return_sum)
         xc, other = _aligned16(xc), _aligned16(other)

@@ -72,8 +72,10 @@ class BF16RotateLinearWrapper(nn.Module):
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         rl = self.rotate_linear
-        if isinstance(rl, RotateLinearInt4) and isinstance(rl.qlinear, MarlinW4A8Linear):
-            return rl.qlinear.forward_rotated(x, rl.rotation, input_fp16=True, out_dtype=x.dtype)
+        if isinstance(rl, RotateLinearInt4):
+            q = rl.qlinear
+            if isinstance(q, MarlinW4A8Linear):
+                return q.forward_rotated(x, rl.rotation, input_fp16=True, out_dtype=x.dtype)
         input_dtype = x.dtype
         with torch.amp.autocast("cuda", enabled=False):
             out = rl(x.to(torch.float16))
@@ -394,21 +396,27 @@ class MarlinW4A8Linear(nn.Module):
         y = torch.ops.paroquant.w4a8_gemm(xq, xs, self.qweight, self.scales, self.bias, x.dtype)
         return y.view(*shape[:-1], self.out_features)
 
-    @torch.no_grad()
     def forward_rotated(self, x: torch.Tensor, rotation: Rotation, input_fp16: bool, out_dtype: torch.dtype,
                         materialize_fp16: bool = True) -> torch.Tensor:
         """Rotation + int8 quant + GEMM on un-rotated activations x [..., K].  Eagerly it checks that the
         weights are loaded and (re)prepares the rotation's operands when they are stale; under torch.compile
         it expects a prepared rotation (prepare(), or one eager call)."""
+        bias = self.bias
+        if torch.is_grad_enabled() and (x.requires_grad or (bias is not None and bias.requires_grad)):
+            with torch.no_grad():   # entered only where there is something to record
+                return self.forward_rotated(x, rotation, input_fp16, out_dtype, materialize_fp16)
         if self.in_features > _FUSED_MAX_K:
-            return self._forward_unfused(x, rotation, input_fp16, out_dtype, materialize_fp16)
+            with torch.no_grad():
+                return self._forward_unfused(x, rotation, input_fp16, out_dtype, materialize_fp16)
+        weights = self.qweight
         if not torch.compiler.is_compiling():
-            self._check_loaded()
+            if weights.numel() == 0:
+                self._check_loaded()
             if not rotation.prepared:
                 rotation.prepare()
         return torch.ops.paroquant.w4a8_linear(
-            x, rotation.rot_idx, rotation.rot_cs, rotation.scales_f32, rotation.krot, self.qweight, self.scales,
-            self.bias, input_fp16, materialize_fp16, out_dtype)
+            x, rotation.rot_idx, rotation.rot_cs, rotation.scales_f32, rotation.krot, weights, self.scales,
+            bias, input_fp16, materialize_fp16, out_dtype)
 
     def _forward_unfused(self, x, rotation, input_fp16, out_dtype, materialize_fp16):
         """The same computation as paroquant::w4a8_linear in three ops, for rows longer than its kernels take

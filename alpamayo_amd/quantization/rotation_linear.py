@@ -114,7 +114,19 @@ class Rotation(nn.Module):
         False again after load_state_dict, an in-place update or a move of any of them.  Buffers created under
         torch.inference_mode() carry no version counter, so only a replacement or a move of them is seen:
         after changing such a buffer in place, call prepare()."""
-        return self.rot_cs.numel() > 0 and self._prep_src == self._param_source()
+        src = self._prep_src
+        if src is None or self.rot_cs.numel() == 0:
+            return False
+        # what ops.tensor_state() says of each, compared in place (this runs on every eager call)
+        for t, (ptr, ver, dev) in zip((self.theta, self.pairs, self.channel_scales), src):
+            if t is None or t.data_ptr() != ptr or t.device != dev:
+                return False
+            if t.is_inference():
+                if ver is not None:
+                    return False
+            elif t._version != ver:
+                return False
+        return True
 
 
 class RotateLinearInt4(nn.Module):
