@@ -129,6 +129,20 @@ __host__ __device__ __forceinline__ int64_t a_tile_offset(int64_t row, int k, in
 }
 
 // ---------------------------------------------------------------------------
+// Tiled fp16 activations, m * k values: row blocks of 16 rows, each
+// [G][4][4][r][8] with r its rows (16, or m % 16 in a ragged last block).  Part
+// (g, q, j, c) holds values 128 g + 32 j + 8 q .. + 7 of the block's row c: what
+// lane 16 j + c of v_mfma_f32_16x16x32_f16 multiplies with dword q of its packed
+// weights, so a fragment of a full block is one contiguous 1 KB load.
+// ---------------------------------------------------------------------------
+__host__ __device__ __forceinline__ int64_t a16_tile_offset(int64_t row, int k, int64_t m, int G) {
+  const int64_t r0 = row & ~static_cast<int64_t>(15);
+  const int r = m - r0 < 16 ? static_cast<int>(m - r0) : 16;
+  return r0 * G * 128 + ((k >> 7) * 128 + ((k >> 3) & 3) * 32 + ((k >> 5) & 3) * 8) * r +
+         static_cast<int>(row - r0) * 8 + (k & 7);
+}
+
+// ---------------------------------------------------------------------------
 // int4 weight unpacking (layout in pq_gemm.hip): a dword of 8 codes -> two
 // dwords of 4 signed bytes (q - z).  Every byte stays in [113, 143] before the
 // xor, so no carry crosses a byte; the xor maps 128 + d to two's complement d.

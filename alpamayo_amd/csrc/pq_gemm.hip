@@ -950,7 +950,7 @@ void launch_prefill(const pq::GemmGroup& grp, int bias_dtype, int y_dtype, int M
 // ---------------------------------------------------------------------------
 // Host-side configuration
 // ---------------------------------------------------------------------------
-// The decode GEMM on int8 A takes up to 64 rows, all its row blocks of 16
+// The decode GEMM on row-major int8 A takes up to 64 rows, all its row blocks of 16
 // in every workgroup (the weights are read once): the grouped decode layer at
 // M = 33-64 on it against the row rotate+quant kernel and the prefill GEMM's
 // tiles is recorded in the design notes.

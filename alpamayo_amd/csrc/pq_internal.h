@@ -54,7 +54,8 @@ struct RotMember {
 struct RotGroup {
   RotMember mem[kMaxGroup];
   int count;
-  int tiled;   // row kernel: rows m of the tiled order (pqd::a_tile_offset) for the int8 codes; 0: row-major
+  int tiled;   // row kernel: rows m of the tiled order (pqd::a_tile_offset, a16_tile_offset) of the int8 codes
+               // and of the fp16 rows; 0: row-major
 };
 
 // Per-token int8 quantization of a split rotation's output (launch_quant_split):

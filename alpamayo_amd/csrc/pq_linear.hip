@@ -11,10 +11,11 @@
 //     are already in flight.
 //   split3 (k >= 4096 beyond that, up to 64 tokens): the split rotation
 //     with the rows spread over waves, a token-scale + int8 kernel, then
-//     the decode GEMM on int8 A (three launches).
+//     the decode GEMM on int8 A (three launches; from 17 rows the mid-size
+//     GEMM, for which the codes are written tiled).
 //   rows (otherwise): pq_rotate_quant_i8 (rotation + absmax + int8 quant of
-//     whole rows per workgroup) into the caller's workspace, then
-//     pq_w4a8_gemm.
+//     whole rows per workgroup) into the caller's workspace, then the
+//     mid-size GEMM (17 to 512 rows) or the kernels of pq_w4a8_gemm.
 //
 // A one-kernel variant (every workgroup rotating the token itself) was
 // measured slower: the K/128 x 5 KB of rotation parameters, re-read by each

@@ -369,7 +369,8 @@ __global__ __launch_bounds__(kRQWaves * 64) void rotate_quant_kernel(const void*
           uint32_t w[4];
 #pragma unroll
           for (int m = 0; m < 4; ++m) w[m] = pqd::f16_pair(d, 2 * m * RB + r, (2 * m + 1) * RB + r);
-          *reinterpret_cast<uint4*>(xrot + ro) = make_uint4(w[0], w[1], w[2], w[3]);
+          *reinterpret_cast<uint4*>(xrot + (grp.tiled ? pqd::a16_tile_offset(row0 + r, c8, grp.tiled, G) : ro)) =
+              make_uint4(w[0], w[1], w[2], w[3]);
         }
         if (xq != nullptr) {
           const float inv = s_inv[r];
@@ -402,7 +403,8 @@ __global__ __launch_bounds__(kRQWaves * 64) void rotate_quant_kernel(const void*
         o.y = pqd::pk_f16(f[2], f[3]);
         o.z = pqd::pk_f16(f[4], f[5]);
         o.w = pqd::pk_f16(f[6], f[7]);
-        *reinterpret_cast<uint4*>(xrot + (row0 + r) * h + c8) = o;
+        *reinterpret_cast<uint4*>(xrot + (grp.tiled ? pqd::a16_tile_offset(row0 + r, c8, grp.tiled, G)
+                                                    : (row0 + r) * h + c8)) = o;
       }
       if (xq != nullptr) {
         uint2 o;

@@ -25,11 +25,13 @@
 // are complete after that: no per-group epilogue, the MFMA accumulators run
 // over all of K.
 //
-// Two kernels:
+// Kernels:
 //   w16_skinny   M <= 16: as the W4A8 decode GEMM (waves split K by groups,
 //                fixed-order LDS sum of their partials), four
 //                v_mfma_f32_16x16x32_f16 per 1 KB weight block, A rows read
 //                from memory (rows past M repeat row M-1, never stored).
+//   w16_mid      17 to 512 rows behind the linear entry points, until the prefill
+//                tiles fill the chip: pq_w4a16_mid.h.
 //   w16_prefill  M > 16: 192x256 (or 128x128) tiles, 8 (or 4) waves side by
 //                side along n, v_mfma_f32_32x32x16_f16.  A stage of the LDS
 //                ring is half a K group (64 k): BM rows x 128 B of A
@@ -41,49 +43,13 @@
 
 #include "pq_device.h"
 #include "pq_internal.h"
+#include "pq_w4a16.h"
 
 using namespace pqd;
 
-typedef _Float16 v2h __attribute__((ext_vector_type(2)));
-typedef _Float16 v8h __attribute__((ext_vector_type(8)));
-typedef float v4f __attribute__((ext_vector_type(4)));
-typedef float v16f __attribute__((ext_vector_type(16)));
+using namespace pqw16;
 
 namespace {
-
-struct W16Args {
-  const uint16_t* x;       // fp16 [m][k]
-  const uint8_t* wpack;    // packed codes
-  const uint32_t* wmeta;   // s | sz << 16 per (tile, group, column)
-  const void* bias;        // [n] or null
-  void* y;                 // [m][n]
-  int n;
-};
-
-__device__ __forceinline__ v2h as_h2(uint32_t u) { return __builtin_bit_cast(v2h, u); }
-__device__ __forceinline__ uint32_t as_u32(v2h h) { return __builtin_bit_cast(uint32_t, h); }
-
-// fp16 pairs {s, s} and {sz, sz} of a metadata word.
-__device__ __forceinline__ v2h meta_s2(uint32_t meta) { return as_h2(__builtin_amdgcn_perm(meta, meta, 0x01000100u)); }
-__device__ __forceinline__ v2h meta_z2(uint32_t meta) { return as_h2(__builtin_amdgcn_perm(meta, meta, 0x03020302u)); }
-
-// One dword of codes (k order: the low nibbles of bytes 0..3, then the high
-// nibbles) -> its 8 weights fp16(q * s + sz), in k order.
-__device__ __forceinline__ v8h dequant8(uint32_t w, v2h s2, v2h z2) {
-  const uint32_t lo = w & 0x0f0f0f0fu;
-  const uint32_t hi = (w >> 4) & 0x0f0f0f0fu;
-  // selector bytes 0..3 pick bytes of the second operand, 4 picks 0x64:
-  // halves 0x6400 + q = 1024 + q
-  constexpr uint32_t kE = 0x64646464u;
-  const v2h off = {static_cast<_Float16>(1024.0f), static_cast<_Float16>(1024.0f)};
-  const v2h q01 = as_h2(__builtin_amdgcn_perm(kE, lo, 0x04010400u)) - off;
-  const v2h q23 = as_h2(__builtin_amdgcn_perm(kE, lo, 0x04030402u)) - off;
-  const v2h q45 = as_h2(__builtin_amdgcn_perm(kE, hi, 0x04010400u)) - off;
-  const v2h q67 = as_h2(__builtin_amdgcn_perm(kE, hi, 0x04030402u)) - off;
-  const uint4 r = {as_u32(__builtin_elementwise_fma(q01, s2, z2)), as_u32(__builtin_elementwise_fma(q23, s2, z2)),
-                   as_u32(__builtin_elementwise_fma(q45, s2, z2)), as_u32(__builtin_elementwise_fma(q67, s2, z2))};
-  return __builtin_bit_cast(v8h, r);
-}
 
 // ---------------------------------------------------------------------------
 // Decode-size GEMM (M <= 16)
@@ -94,14 +60,6 @@ __device__ __forceinline__ v8h dequant8(uint32_t w, v2h s2, v2h z2) {
 // them each, against the same 8 k of A row c (one 16-byte load each).
 // ---------------------------------------------------------------------------
 constexpr int kW16SkinnyRows = 16;
-
-// Linears that share their input, as one decode GEMM launch: member i owns
-// workgroups first[i] .. first[i+1]-1 (set by the launcher).
-struct W16Group {
-  W16Args mem[pq::kMaxGroup];
-  int first[pq::kMaxGroup + 1];
-  int count;
-};
 
 template <int NT, int W, int U>
 __global__ __launch_bounds__(W * 64) void w16_skinny(const W16Group grp, int bias_dtype, int y_dtype, int M, int K) {
@@ -595,11 +553,15 @@ int w16_linear_group(const char* who, const void* x, int x_dtype, const pq_linea
   }
   const unsigned rflags = flags | PQ_RQ_MATERIALIZE_FP16;
   // One row per wave, as the W4A8 linear's split rotation.
+  // The mid-size GEMM reads the fp16 rows in the tiled order, which the row kernel then writes.
+  const bool mid = !split && w16_mid_takes(gg, m, k);
+  rg.tiled = mid ? M : 0;
   if (split) pq::launch_rotate_split(x, x_dtype, rg, M, K, krot, rflags, s, norm, 1);
   else pq::launch_rotate_quant_group(x, x_dtype, rg, m, K, krot, rflags, s, norm);
   int st = pq::launch_status("W4A16 linear rotation launch");
   if (st != PQ_OK) return st;
-  launch_w16_gemm_group(gg, bias_dtype, y_dtype, M, K, s);
+  if (mid) launch_w16_mid(gg, bias_dtype, y_dtype, M, K, s);
+  else launch_w16_gemm_group(gg, bias_dtype, y_dtype, M, K, s);
   return pq::launch_status("W4A16 linear GEMM launch");
 }
 

@@ -107,7 +107,7 @@ class SharedInputRotateLinears(nn.Module):
     rotation + quant launch for all members and one GEMM launch over their
     concatenated output columns, where separate calls take two launches per
     linear) or all WQLinear weights (W4A16: paroquant::w4a16_linear_group,
-    one rotation launch and, up to 16 tokens, one GEMM launch).  The reference
+    one rotation launch and, at decode and mid sizes, one GEMM launch).  The reference
     keeps these linears separate once ParoQuant is loaded
     (paroquant_marlin_w4a8.py:455-460); its unquantised counterparts are
     QKVLinear / MergedColumnLinear (patches.py:144-263).
