@@ -501,7 +501,7 @@ __device__ __forceinline__ void wait_groups(int ahead) {
 }
 
 // CLS > 1: the sum over the groups is taken in CLS chains, chain c over groups
-// c, c + CLS, ..., then ((chain 0 + chain 1) + ...): the order in which the
+// c G / CLS .. (c + 1) G / CLS - 1, then ((chain 0 + chain 1) + ...): the order in which the
 // mid-size GEMM adds the partial sums of CLS waves, so that a row's outputs
 // have the same bits on either kernel.  One more set of accumulators.
 template <int BM, int BN, int WM, int WN, bool PARTIALS, int ST = kPfStages, bool TP = false, int CLS = 1>
@@ -596,11 +596,11 @@ __global__ __launch_bounds__(WM * WN * 64) void gemm_prefill(
 #pragma unroll
   for (int tn = 0; tn < TN; ++tn) bcol[tn] = wn * (BN / WN) + tn * 32 + r32;
 
-  // Matrix work of group g from its stage.  The loads of step ig (two ahead, group gi)
+  // Matrix work of group g from its stage.  The loads of group ig (= g + 2)
   // are issued after the first two k-steps' MFMAs: issued at the top of the
   // group, right after the barrier, all waves' copies queue up at once in
   // the load path while no MFMA is in flight.
-  auto compute = [&](int stage, int g, int ig, int gi) {
+  auto compute = [&](int stage, int g, int ig) {
     const uint8_t* As = smem + stage * STAGE;
     const uint8_t* Bs = As + A_BYTES;
     const uint32_t* Ms = reinterpret_cast<const uint32_t*>(Bs + B_BYTES);
@@ -636,7 +636,7 @@ __global__ __launch_bounds__(WM * WN * 64) void gemm_prefill(
 #pragma unroll
         for (int tn = 0; tn < TN; ++tn)
           T[tm][tn] = __builtin_amdgcn_mfma_i32_32x32x32_i8(a[tm], b[tn], T[tm][tn], 0, 0, 0);
-      if (i == 1 && ig < G) issue(gi, ig % ST);
+      if (i == 1 && ig < G) issue(ig, ig % ST);
     }
     if constexpr (PARTIALS) {
 #pragma unroll
@@ -672,7 +672,7 @@ __global__ __launch_bounds__(WM * WN * 64) void gemm_prefill(
     const int n = bn * BN + bcol[tn];
     if (m < M && n < N) partials[(m * G + g) * N + n] = val;
   };
-  auto compute_tp = [&](int stage, int g, int ig, int gi) {
+  auto compute_tp = [&](int stage, int g, int ig) {
     static_assert(!TP || TM % 2 == 0, "tiles in pairs");
     const uint8_t* As = smem + stage * STAGE;
     const uint8_t* Bs = As + A_BYTES;
@@ -739,7 +739,7 @@ __global__ __launch_bounds__(WM * WN * 64) void gemm_prefill(
           __builtin_amdgcn_sched_group_barrier(0x002, 8, 0);   // eight VALU
         }
       }
-      if (p == 0 && ig < G) issue(gi, ig % ST);
+      if (p == 0 && ig < G) issue(ig, ig % ST);
     }
     constexpr int LP = (TM / 2 - 1) & 1;
 #pragma unroll
@@ -765,25 +765,21 @@ __global__ __launch_bounds__(WM * WN * 64) void gemm_prefill(
     lds_copy4(xs + min(bm * BM + r, M - 1), lds0 + ST * STAGE + wave * 256);
   }
   static_assert(LOADS * (ST - 2) < 64, "vmcnt range");
-  // Step i computes the i-th group of the order: ascending, or chain by chain.
-  auto after = [&](int g) { return CLS == 1 || g + CLS < G ? g + CLS : g % CLS + 1; };
   float tot[CLS > 1 ? TM : 1][TN][16];
-  int gq = 0;   // the next group to copy
+  int chain = 0, chain_end = G / CLS;
 #pragma unroll
   for (int q = 0; q < ST - 1; ++q)
-    if (q < G) {
-      issue(gq, q);
-      gq = after(gq);
-    }
-  int g = 0;
-  for (int i = 0; i < G; ++i) {
-    wait_groups<LOADS, ST - 2>(min(G - 1 - i, ST - 2));
+    if (q < G) issue(q, q);
+  for (int g = 0; g < G; ++g) {
+    wait_groups<LOADS, ST - 2>(min(G - 1 - g, ST - 2));
     __builtin_amdgcn_s_barrier();
-    if constexpr (TP) compute_tp(i % ST, g, i + ST - 1, gq);
-    else compute(i % ST, g, i + ST - 1, gq);
+    if constexpr (TP) compute_tp(g % ST, g, g + ST - 1);
+    else compute(g % ST, g, g + ST - 1);
     if constexpr (CLS > 1) {
-      if (g + CLS >= G) {   // the chain's last group
-        const bool first = g % CLS == 0;
+      if (g + 1 == chain_end) {   // the chain's last group (no chain is empty: G >= CLS)
+        const bool first = chain == 0;
+        ++chain;
+        chain_end = (chain + 1) * G / CLS;
 #pragma unroll
         for (int tm = 0; tm < TM; ++tm)
 #pragma unroll
@@ -795,8 +791,6 @@ __global__ __launch_bounds__(WM * WN * 64) void gemm_prefill(
             }
       }
     }
-    g = after(g);
-    gq = after(gq);
   }
   if constexpr (PARTIALS) return;
   if constexpr (CLS > 1) {
@@ -1095,8 +1089,14 @@ bool gemm_rotated_supported(int64_t m, int64_t k) {
 
 void launch_gemm_chains(const GemmGroup& grp, int chains, int bias_dtype, int y_dtype, int m, int k,
                         hipStream_t stream) {
+  int64_t tiles = 0;
+  for (int i = 0; i < grp.count; ++i) tiles += (grp.mem[i].n + 255) / 256;
+  tiles *= (m + 127) / 128;
   if (chains == 8) launch_prefill_t<128, 256, 1, 8, false, kPfStages, true, 8>(grp, bias_dtype, y_dtype, m, k, stream);
-  else launch_prefill_t<128, 256, 1, 8, false, kPfStages, true, 4>(grp, bias_dtype, y_dtype, m, k, stream);
+  else if (tiles >= 128)
+    launch_prefill_t<128, 256, 1, 8, false, kPfStages, true, 4>(grp, bias_dtype, y_dtype, m, k, stream);
+  else   // as launch_prefill: half-size tiles where the big ones leave half of the CUs idle
+    launch_prefill_t<128, 128, 1, 4, false, kPfStages, false, 4>(grp, bias_dtype, y_dtype, m, k, stream);
 }
 
 void launch_gemm_group(GemmGroup grp, int aq, int bias_dtype, int y_dtype, int m, int k, hipStream_t stream) {

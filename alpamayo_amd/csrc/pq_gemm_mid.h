@@ -3,8 +3,8 @@
 // Between the decode sizes (every wave streams its weights once, A is tiny)
 // and the prefill sizes (big LDS tiles shared by a workgroup) a launch has
 // too few big tiles to fill the chip and too many rows for one row block.
-// Here a wave owns RB x NT blocks of 16 x 16 outputs and walks every WK-th
-// 128-group of K on its own: operands go from memory straight into
+// Here a wave owns RB x NT blocks of 16 x 16 outputs and walks one of
+// WK parts of K on its own: operands go from memory straight into
 // registers, two groups ahead, and no wave waits for another until the WK
 // partial sums of a workgroup meet in LDS at the end (added in a fixed
 // order).  No barrier in the K loop, so the waves of a SIMD drift apart and
@@ -158,11 +158,11 @@ __global__ __launch_bounds__(WK * WN * 64) void gemm_mid(const pq::GemmGroup grp
     }
   };
 
-  // Wave wk walks groups wk, wk + WK, ...: n of them (the host keeps WK <= G).
+  // Wave wk walks the n groups of its part of K (the host keeps WK <= G).
   // Two register stages; the tail is peeled so that no load sits behind a
   // branch (the compiler would wait for every load at the join).
-  const int n = (G - wk + WK - 1) / WK;
-  auto grp_of = [&](int i) { return wk + i * WK; };
+  const int gb = wk * G / WK, n = (wk + 1) * G / WK - gb;
+  auto grp_of = [&](int i) { return gb + i; };
   Stage<RB, NT> s0, s1;
   load(s0, grp_of(0));
   load(s1, grp_of(min(1, n - 1)));

@@ -15,7 +15,7 @@ struct MidCfg {
 // times the groups each wave walks (G / WK, written as 8 / WK since G is
 // common to all), and the launch takes ceil(workgroups / 256) of them.  Ties
 // go to more columns per workgroup (fewer partial sums through LDS).  One
-// column tile per wave where two would use half of the CUs (up to 32 rows).
+// column tile per wave where two would leave CUs idle (up to 128 rows).
 // Past kMidFixedRows rows WK is gemm_chains(m).
 // Measured against the row-major 16-row-block kernel and the LDS-tile kernel,
 // weights from HBM (us, before -> after):
@@ -25,9 +25,6 @@ struct MidCfg {
 //   N = 24576, K = 4096:  M = 32 19.0 -> 16.7, 64 41.3 -> 22.1, 96 35.3 -> 30.9
 MidCfg choose_mid(const pq::GemmGroup& grp, int m) {
   const int nrb = (m + 15) / 16;
-  int64_t tiles = 0;
-  for (int i = 0; i < grp.count; ++i) tiles += grp.mem[i].n / 16;
-  if (nrb <= 2 && tiles <= 256) return {2, 1, 8, 1};
   MidCfg best{0, 0, 0, 0};
   int64_t best_cost = 0;
   auto consider = [&](int rb, int nt, int wn) {
@@ -45,6 +42,7 @@ MidCfg choose_mid(const pq::GemmGroup& grp, int m) {
     if (m > pq::kMidFixedRows && wn < 4) consider(3, 4, wn);
     for (int rb = 2; rb <= 4; ++rb) consider(rb, 2, wn);
   }
+  consider(2, 1, 1);
   return best;
 }
 
@@ -88,7 +86,7 @@ namespace pq {
 // as fast on row-major A) to kMidMaxRows, with at least 8 groups of K, one per
 // wave.  Past 2.8 M outputs, 11 K per CU, the LDS tiles of the prefill kernel,
 // which share each operand over a workgroup, win where 128 x 256 tiles fill
-// half of the CUs (N = 24576: M = 96 30.9 against 35.3 us, M = 128 35.2
+// half of the CUs, and past 3.2 M outputs its 128 x 128 tiles (N = 24576: M = 96 30.9 against 35.3 us, M = 128 35.2
 // against 32.4, M = 200 53 against 42; N = 4096, K = 4096: M = 512 20.4
 // against 24.6, M = 800 33 against 31).
 MidGemm gemm_mid_choice(const GemmGroup& grp, int64_t m, int64_t k) {
@@ -98,7 +96,8 @@ MidGemm gemm_mid_choice(const GemmGroup& grp, int64_t m, int64_t k) {
     n += grp.mem[i].n;
     tiles256 += (grp.mem[i].n + 255) / 256;
   }
-  if (m > kMidFixedRows && (m + 15) / 16 * 16 * n > 2800000 && (m + 127) / 128 * tiles256 >= 128)
+  const int64_t outputs = (m + 15) / 16 * 16 * n;
+  if (m > kMidFixedRows && outputs > 2800000 && ((m + 127) / 128 * tiles256 >= 128 || (m > 128 && outputs > 3200000)))
     return MidGemm::kChains;
   return MidGemm::kTiled;
 }

@@ -36,6 +36,7 @@ pytestmark = pytest.mark.gpu
     (511, 1024, (1040,), (True, True)),          # the most rows it takes, less one
     (160, 1152, (12288, 12304), (True, True)),   # too wide: the prefill tiles in four chains of K
     (113, 1408, (24576,), (True, True)),         # in eight chains
+    (500, 1152, (6144, 1280), (True, True)),     # 128 x 128 tiles in four chains
 ])
 def test_tiled_gemm(M, K, ns, flags):
     print(f"tiled GEMM M={M} K={K} ns={ns} flags={flags}", flush=True)
