@@ -502,8 +502,9 @@ __device__ __forceinline__ void wait_groups(int ahead) {
 
 // CLS > 1: the sum over the groups is taken in CLS chains, chain c over groups
 // c G / CLS .. (c + 1) G / CLS - 1, then ((chain 0 + chain 1) + ...): the order in which the
-// mid-size GEMM adds the partial sums of CLS waves, so that a row's outputs
-// have the same bits on either kernel.  One more set of accumulators.
+// mid-size GEMM adds the partial sums of CLS = kMidChains waves (of eight it
+// adds them in pairs first), so that a row's outputs have the same bits on
+// either kernel.  One more set of accumulators.
 template <int BM, int BN, int WM, int WN, bool PARTIALS, int ST = kPfStages, bool TP = false, int CLS = 1>
 __global__ __launch_bounds__(WM * WN * 64) void gemm_prefill(
     const pq::GemmGroup grp, int bias_dtype, int y_dtype, int M, int K) {
@@ -1087,16 +1088,14 @@ bool gemm_rotated_supported(int64_t m, int64_t k) {
   return m >= 1 && m <= kSkinnyRows && k % 128 == 0 && k <= 16384 && m * (k + 16) <= 80 * 1024;
 }
 
-void launch_gemm_chains(const GemmGroup& grp, int chains, int bias_dtype, int y_dtype, int m, int k,
-                        hipStream_t stream) {
+void launch_gemm_chains(const GemmGroup& grp, int bias_dtype, int y_dtype, int m, int k, hipStream_t stream) {
   int64_t tiles = 0;
   for (int i = 0; i < grp.count; ++i) tiles += (grp.mem[i].n + 255) / 256;
   tiles *= (m + 127) / 128;
-  if (chains == 8) launch_prefill_t<128, 256, 1, 8, false, kPfStages, true, 8>(grp, bias_dtype, y_dtype, m, k, stream);
-  else if (tiles >= 128)
-    launch_prefill_t<128, 256, 1, 8, false, kPfStages, true, 4>(grp, bias_dtype, y_dtype, m, k, stream);
+  if (tiles >= 128)
+    launch_prefill_t<128, 256, 1, 8, false, kPfStages, true, kMidChains>(grp, bias_dtype, y_dtype, m, k, stream);
   else   // as launch_prefill: half-size tiles where the big ones leave half of the CUs idle
-    launch_prefill_t<128, 128, 1, 4, false, kPfStages, false, 4>(grp, bias_dtype, y_dtype, m, k, stream);
+    launch_prefill_t<128, 128, 1, 4, false, kPfStages, false, kMidChains>(grp, bias_dtype, y_dtype, m, k, stream);
 }
 
 void launch_gemm_group(GemmGroup grp, int aq, int bias_dtype, int y_dtype, int m, int k, hipStream_t stream) {

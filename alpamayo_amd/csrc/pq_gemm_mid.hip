@@ -16,7 +16,7 @@ struct MidCfg {
 // common to all), and the launch takes ceil(workgroups / 256) of them.  Ties
 // go to more columns per workgroup (fewer partial sums through LDS).  One
 // column tile per wave where two would leave CUs idle (up to 128 rows).
-// Past kMidFixedRows rows WK is gemm_chains(m).
+// Past kMidFixedRows rows WK is gemm_mid_waves(m).
 // Measured against the row-major 16-row-block kernel and the LDS-tile kernel,
 // weights from HBM (us, before -> after):
 //   N = 4096, K = 4096:   M = 32 7.5 -> 5.5, 64 12.5 -> 6.4, 128 18.1 -> 8.1, 200 18.5 -> 11.4, 512 24.6 -> 20.4
@@ -28,7 +28,7 @@ MidCfg choose_mid(const pq::GemmGroup& grp, int m) {
   MidCfg best{0, 0, 0, 0};
   int64_t best_cost = 0;
   auto consider = [&](int rb, int nt, int wn) {
-    if (m > pq::kMidFixedRows && 8 / wn != pq::gemm_chains(m)) return;
+    if (m > pq::kMidFixedRows && 8 / wn != pq::gemm_mid_waves(m)) return;
     int64_t units = 0;
     for (int i = 0; i < grp.count; ++i) units += (grp.mem[i].n / 16 + nt * wn - 1) / (nt * wn);
     const int64_t wgs = units * ((nrb + rb - 1) / rb);
@@ -97,7 +97,8 @@ MidGemm gemm_mid_choice(const GemmGroup& grp, int64_t m, int64_t k) {
     tiles256 += (grp.mem[i].n + 255) / 256;
   }
   const int64_t outputs = (m + 15) / 16 * 16 * n;
-  if (m > kMidFixedRows && outputs > 2800000 && ((m + 127) / 128 * tiles256 >= 128 || (m > 128 && outputs > 3200000)))
+  if (gemm_mid_waves(m) == kMidChains && m > kMidFixedRows && outputs > 2800000 &&
+      ((m + 127) / 128 * tiles256 >= 128 || outputs > 3200000))
     return MidGemm::kChains;
   return MidGemm::kTiled;
 }

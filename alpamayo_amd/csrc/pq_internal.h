@@ -144,22 +144,19 @@ PQ_HIDDEN void launch_gemm_group(GemmGroup grp, int aq, int bias_dtype, int y_dt
 // A image and token scales) go to the member's partials / a_out / as_out.
 PQ_HIDDEN void launch_gemm_group_partials(GemmGroup grp, int aq, int m, int k, hipStream_t stream);
 
-// The GEMM of a group on tiled int8 codes (xq in the order of
-// pqd::a_tile_offset): whether it is the one
-// to run for m rows and n_total output columns, and its launches.
+// The GEMM behind the quantizers of a group of m rows: kNone that of launch_gemm_group, kTiled the mid-size GEMM on
+// tiled int8 codes (xq in the order of pqd::a_tile_offset), kChains the prefill tiles on row-major codes, summing in
+// the mid-size GEMM's order.
 //
-// From kMidFixedRows + 1 rows on, a row's outputs must not depend on which
-// linears share its launch (a group returns the bits its members return when
-// called one by one), so the order of the sum over K is fixed by m: 8 chains
-// up to 128 rows, 4 above (gemm_chains), whatever the number of columns; a
-// launch too wide for the mid-size GEMM then runs the prefill tiles with the
-// same chains (launch_gemm_chains, row-major codes).
-constexpr int kMidFixedRows = 64, kMidMaxRows = 512;
+// From kMidFixedRows + 1 rows on, a row's outputs must not depend on which linears share its launch (a group
+// returns the bits its members return when called one by one), so there the order of the sum over K is fixed by m
+// (gemm_mid_waves: the waves of the mid-size GEMM that split K).  The prefill tiles can take the place of its
+// kMidChains waves, not of eight, which are for few rows.
+constexpr int kMidFixedRows = 64, kMidMaxRows = 512, kMidChains = 4;
+constexpr int gemm_mid_waves(int64_t m) { return m <= 128 ? 8 : kMidChains; }
 enum class MidGemm { kNone, kTiled, kChains };
 PQ_HIDDEN MidGemm gemm_mid_choice(const GemmGroup& grp, int64_t m, int64_t k);
-constexpr int gemm_chains(int64_t m) { return m <= 128 ? 8 : 4; }
-PQ_HIDDEN void launch_gemm_chains(const GemmGroup& grp, int chains, int bias_dtype, int y_dtype, int m, int k,
-                                  hipStream_t stream);
+PQ_HIDDEN void launch_gemm_chains(const GemmGroup& grp, int bias_dtype, int y_dtype, int m, int k, hipStream_t stream);
 PQ_HIDDEN void launch_gemm_mid(const GemmGroup& grp, int bias_dtype, int y_dtype, int m, int k, hipStream_t stream);
 PQ_HIDDEN void launch_gemm_mid_partials(const GemmGroup& grp, int m, int k, hipStream_t stream);
 // Row-major copy [m][k] of tiled codes.

@@ -214,7 +214,7 @@ int linear_group(const char* who, const void* x, int x_dtype, const pq_linear_me
   const int aq = path == Path::kSplit ? (mat16 ? 1 : 2) : 0;
   if (probe == nullptr && mid != pq::MidGemm::kNone) {
     if (tiled) pq::launch_gemm_mid(gg, bias_dtype, y_dtype, M, K, s);
-    else pq::launch_gemm_chains(gg, pq::gemm_chains(M), bias_dtype, y_dtype, M, K, s);
+    else pq::launch_gemm_chains(gg, bias_dtype, y_dtype, M, K, s);
     return pq::launch_status("linear GEMM launch");
   }
   if (probe == nullptr) {

@@ -35,7 +35,9 @@ pytestmark = pytest.mark.gpu
     (255, 1024, (5120,), (True, True)),
     (511, 1024, (1040,), (True, True)),          # the most rows it takes, less one
     (160, 1152, (12288, 12304), (True, True)),   # too wide: the prefill tiles in four chains of K
-    (113, 1408, (24576,), (True, True)),         # in eight chains
+    (113, 1408, (24576,), (True, True)),         # one wide member: the widest launch of the tiled kernel itself
+    (96, 1152, (16384, 16400), (True, True)),    # a group too wide for one round, each member in less than one
+    (113, 1408, (8192,) * 4, (True, True)),
     (500, 1152, (6144, 1280), (True, True)),     # 128 x 128 tiles in four chains
 ])
 def test_tiled_gemm(M, K, ns, flags):
