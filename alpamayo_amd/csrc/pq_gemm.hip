@@ -1088,14 +1088,24 @@ bool gemm_rotated_supported(int64_t m, int64_t k) {
   return m >= 1 && m <= kSkinnyRows && k % 128 == 0 && k <= 16384 && m * (k + 16) <= 80 * 1024;
 }
 
-void launch_gemm_chains(const GemmGroup& grp, int bias_dtype, int y_dtype, int m, int k, hipStream_t stream) {
+template <bool PARTIALS>
+void launch_chains(const GemmGroup& grp, int bias_dtype, int y_dtype, int m, int k, hipStream_t stream) {
+  constexpr int C = PARTIALS ? 1 : kMidChains;   // the int32 partials are stored before any sum
   int64_t tiles = 0;
   for (int i = 0; i < grp.count; ++i) tiles += (grp.mem[i].n + 255) / 256;
   tiles *= (m + 127) / 128;
   if (tiles >= 128)
-    launch_prefill_t<128, 256, 1, 8, false, kPfStages, true, kMidChains>(grp, bias_dtype, y_dtype, m, k, stream);
+    launch_prefill_t<128, 256, 1, 8, PARTIALS, kPfStages, true, C>(grp, bias_dtype, y_dtype, m, k, stream);
   else   // as launch_prefill: half-size tiles where the big ones leave half of the CUs idle
-    launch_prefill_t<128, 128, 1, 4, false, kPfStages, false, kMidChains>(grp, bias_dtype, y_dtype, m, k, stream);
+    launch_prefill_t<128, 128, 1, 4, PARTIALS, kPfStages, false, C>(grp, bias_dtype, y_dtype, m, k, stream);
+}
+
+void launch_gemm_chains(const GemmGroup& grp, int bias_dtype, int y_dtype, int m, int k, hipStream_t stream) {
+  launch_chains<false>(grp, bias_dtype, y_dtype, m, k, stream);
+}
+
+void launch_gemm_chains_partials(const GemmGroup& grp, int m, int k, hipStream_t stream) {
+  launch_chains<true>(grp, 0, 0, m, k, stream);
 }
 
 void launch_gemm_group(GemmGroup grp, int aq, int bias_dtype, int y_dtype, int m, int k, hipStream_t stream) {

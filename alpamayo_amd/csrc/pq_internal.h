@@ -157,6 +157,7 @@ constexpr int gemm_mid_waves(int64_t m) { return m <= 128 ? 8 : kMidChains; }
 enum class MidGemm { kNone, kTiled, kChains };
 PQ_HIDDEN MidGemm gemm_mid_choice(const GemmGroup& grp, int64_t m, int64_t k);
 PQ_HIDDEN void launch_gemm_chains(const GemmGroup& grp, int bias_dtype, int y_dtype, int m, int k, hipStream_t stream);
+PQ_HIDDEN void launch_gemm_chains_partials(const GemmGroup& grp, int m, int k, hipStream_t stream);
 PQ_HIDDEN void launch_gemm_mid(const GemmGroup& grp, int bias_dtype, int y_dtype, int m, int k, hipStream_t stream);
 PQ_HIDDEN void launch_gemm_mid_partials(const GemmGroup& grp, int m, int k, hipStream_t stream);
 // Row-major copy [m][k] of tiled codes.

@@ -243,6 +243,7 @@ int linear_group(const char* who, const void* x, int x_dtype, const pq_linear_me
     }
   }
   if (tiled) pq::launch_gemm_mid_partials(gg, M, K, s);
+  else if (mid == pq::MidGemm::kChains) pq::launch_gemm_chains_partials(gg, M, K, s);
   else pq::launch_gemm_group_partials(gg, aq, M, K, s);
   return pq::launch_status("linear GEMM partials launch");
 }

@@ -2,6 +2,8 @@
 
 from __future__ import annotations
 
+import re
+
 import numpy as np
 import torch
 
@@ -11,6 +13,18 @@ def to_np(t: torch.Tensor) -> np.ndarray:
     if t.dtype == torch.bfloat16:
         t = t.float()
     return t.numpy()
+
+
+def gemm_instances(fn):
+    """(name, template arguments) of the GEMM kernels that one call of fn launches, in launch order."""
+    from torch.profiler import ProfilerActivity, profile
+    fn()
+    torch.cuda.synchronize()
+    with profile(activities=[ProfilerActivity.CUDA]) as prof:
+        fn()
+        torch.cuda.synchronize()
+    found = [re.search(r"(gemm_\w+|w16_\w+)<([^>]*)>", e.name) for e in prof.events()]
+    return [(m[1], tuple(a.strip() for a in m[2].split(","))) for m in found if m]
 
 
 def rel_fro(a, b) -> float:

@@ -14,7 +14,7 @@ import torch
 
 import alpamayo_amd  # noqa: F401
 from alpamayo_amd import workloads
-from tests.gpu_util import to_np
+from tests.gpu_util import gemm_instances, to_np
 from tests.test_gpu_group import _members
 from tests.test_gpu_intermediates import _check, _run
 
@@ -66,3 +66,23 @@ def test_tiled_gemm(M, K, ns, flags):
                                                      torch.float32)
             assert torch.equal(y, single)
         assert torch.equal(y16[i].view(torch.int16), y.to(torch.bfloat16).view(torch.int16))
+
+
+@pytest.mark.parametrize("M,K,ns", [
+    (24, 2048, (4096,)), (80, 2048, (4096, 1040)), (144, 1152, (12288, 12304)), (200, 4096, (8192, 8192)),
+    (500, 1152, (6144, 1280)), (500, 6144, (6144, 1280)),
+])
+def test_parity_form_runs_the_tiles_of_the_product(M, K, ns):
+    """pq_w4a8_linear_group_intermediates multiplies on the kernel and tiling that the linear takes: the same template
+    arguments but for the partials flag and, of gemm_prefill, the chains of the sum that the partials precede, of
+    gemm_mid the cache policy of its weight loads."""
+    print(f"instances M={M} K={K} ns={ns}", flush=True)
+    mbs = _members(ns, K, 8, 5, with_bias=False)
+    x = workloads.activations(M, K, workloads.generator(M)).cuda()
+    get = lambda key: [m[key] for m in mbs]   # noqa: E731
+    args = (get("rot_idx"), get("rot_cs"), get("scales"), 8, get("wp"), get("wm"), get("bias"), True, True)
+    own = {"gemm_prefill": (0, 1, 2, 3, 5, 6), "gemm_mid": (0, 1, 2, 3)}
+    got, want = ([(n, tuple(a[i] for i in own[n])) for n, a in gemm_instances(f)] for f in
+                 (lambda: _run(mbs, x, 8, (True, True)),
+                  lambda: torch.ops.paroquant.w4a8_linear_group(x, *args, torch.bfloat16)))
+    assert want and got == want
