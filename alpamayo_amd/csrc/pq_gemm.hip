@@ -502,9 +502,11 @@ __device__ __forceinline__ void wait_groups(int ahead) {
 
 // CLS > 1: the sum over the groups is taken in CLS chains, chain c over groups
 // c G / CLS .. (c + 1) G / CLS - 1, then ((chain 0 + chain 1) + ...): the order in which the
-// mid-size GEMM adds the partial sums of CLS = kMidChains waves (of eight it
+// mid-size GEMM adds the partial sums of CLS = kMidChains waves (of eight, it
 // adds them in pairs first), so that a row's outputs have the same bits on
-// either kernel.  One more set of accumulators.
+// either kernel.  One more set of accumulators, which 192 x 256 tiles have no
+// registers for (74 spilled: 72 -> 178 us for N = 24576, K = 4096, M = 320);
+// adding a chain costs a launch 2 to 4 us.
 template <int BM, int BN, int WM, int WN, bool PARTIALS, int ST = kPfStages, bool TP = false, int CLS = 1>
 __global__ __launch_bounds__(WM * WN * 64) void gemm_prefill(
     const pq::GemmGroup grp, int bias_dtype, int y_dtype, int M, int K) {
@@ -1088,16 +1090,28 @@ bool gemm_rotated_supported(int64_t m, int64_t k) {
   return m >= 1 && m <= kSkinnyRows && k % 128 == 0 && k <= 16384 && m * (k + 16) <= 80 * 1024;
 }
 
+// The tiles of a launch in chains: 128 x 256 from 160 of them, else 64 x 128 (us with the rotation, K = 4096, M =
+// 224: N = 16384, 128 of them 55.7 against 47.4, N = 24576, 192 of them 58.1 against 68.6).
+int chain_rows(const GemmGroup& grp, int64_t m, int64_t* tiles) {
+  int64_t bn256 = 0, bn128 = 0;
+  for (int i = 0; i < grp.count; ++i) {
+    bn256 += (grp.mem[i].n + 255) / 256;
+    bn128 += (grp.mem[i].n + 127) / 128;
+  }
+  *tiles = (m + 127) / 128 * bn256;
+  if (*tiles >= 160) return 128;
+  *tiles = (m + 63) / 64 * bn128;
+  return 64;
+}
+
 template <bool PARTIALS>
 void launch_chains(const GemmGroup& grp, int bias_dtype, int y_dtype, int m, int k, hipStream_t stream) {
   constexpr int C = PARTIALS ? 1 : kMidChains;   // the int32 partials are stored before any sum
   int64_t tiles = 0;
-  for (int i = 0; i < grp.count; ++i) tiles += (grp.mem[i].n + 255) / 256;
-  tiles *= (m + 127) / 128;
-  if (tiles >= 128)
+  if (chain_rows(grp, m, &tiles) == 128)
     launch_prefill_t<128, 256, 1, 8, PARTIALS, kPfStages, true, C>(grp, bias_dtype, y_dtype, m, k, stream);
-  else   // as launch_prefill: half-size tiles where the big ones leave half of the CUs idle
-    launch_prefill_t<128, 128, 1, 4, PARTIALS, kPfStages, false, C>(grp, bias_dtype, y_dtype, m, k, stream);
+  else
+    launch_prefill_t<64, 128, 1, 4, PARTIALS, kPfStages, false, C>(grp, bias_dtype, y_dtype, m, k, stream);
 }
 
 void launch_gemm_chains(const GemmGroup& grp, int bias_dtype, int y_dtype, int m, int k, hipStream_t stream) {
@@ -1106,6 +1120,15 @@ void launch_gemm_chains(const GemmGroup& grp, int bias_dtype, int y_dtype, int m
 
 void launch_gemm_chains_partials(const GemmGroup& grp, int m, int k, hipStream_t stream) {
   launch_chains<true>(grp, 0, 0, m, k, stream);
+}
+
+double gemm_chains_us(const GemmGroup& grp, int64_t m, int64_t k) {
+  const double g = static_cast<double>(k / 128);
+  int64_t tiles = 0;
+  if (chain_rows(grp, m, &tiles) == 64) return tiles <= 256 ? 0.68 * g : 0.85 * g - 2.0;
+  // rounds of 256 in units of 192 x 256 ones, as launch_prefill counts them
+  const double rounds = 0.71 * static_cast<double>(tiles / 256) + (tiles % 256 != 0 ? 0.64 : 0.0);
+  return rounds * (1.9 * g - 9.0);
 }
 
 void launch_gemm_group(GemmGroup grp, int aq, int bias_dtype, int y_dtype, int m, int k, hipStream_t stream) {

@@ -7,6 +7,7 @@ namespace {
 // split K, WN sit side by side along n, each on RB x NT tiles of 16 x 16.
 struct MidCfg {
   int rb, nt, wk, wn;
+  int64_t cost;   // the busiest CU's, in VALU instructions per wave and 8 groups of K
 };
 
 // The configuration that leaves the busiest CU the least to do.  A wave's
@@ -15,28 +16,24 @@ struct MidCfg {
 // times the groups each wave walks (G / WK, written as 8 / WK since G is
 // common to all), and the launch takes ceil(workgroups / 256) of them.  Ties
 // go to more columns per workgroup (fewer partial sums through LDS).  One
-// column tile per wave where two would leave CUs idle (up to 128 rows).
-// Past kMidFixedRows rows WK is gemm_mid_waves(m).
+// column tile per wave where two would leave CUs idle (eight waves along K).
+// Past kMidFixedRows rows WK is gemm_mid_waves(m, k).
 // Measured against the row-major 16-row-block kernel and the LDS-tile kernel,
 // weights from HBM (us, before -> after):
-//   N = 4096, K = 4096:   M = 32 7.5 -> 5.5, 64 12.5 -> 6.4, 128 18.1 -> 8.1, 200 18.5 -> 11.4, 512 24.6 -> 20.4
+//   N = 4096, K = 4096:   M = 32 7.5 -> 5.5, 64 12.5 -> 6.4, 128 18.1 -> 8.1, 200 18.5 -> 11.4
 //   N = 4096, K = 12288:  M = 32 16.3 -> 11.8, 64 30.1 -> 13.7, 128 47.7 -> 18.9, 200 48.0 -> 27.4, 512 64.9 -> 52.3
-//   N = 6144, K = 4096:   M = 32 7.9 -> 7.2, 64 14.9 -> 9.9, 200 24.2 -> 17.1, 320 24.6 -> 22.9
+//   N = 6144, K = 4096:   M = 32 7.9 -> 7.2, 64 14.9 -> 9.9, 200 24.2 -> 17.1
 //   N = 24576, K = 4096:  M = 32 19.0 -> 16.7, 64 41.3 -> 22.1, 96 35.3 -> 30.9
-MidCfg choose_mid(const pq::GemmGroup& grp, int m) {
+MidCfg choose_mid(const pq::GemmGroup& grp, int m, int k) {
   const int nrb = (m + 15) / 16;
-  MidCfg best{0, 0, 0, 0};
-  int64_t best_cost = 0;
+  MidCfg best{0, 0, 0, 0, 0};
   auto consider = [&](int rb, int nt, int wn) {
-    if (m > pq::kMidFixedRows && 8 / wn != pq::gemm_mid_waves(m)) return;
+    if (m > pq::kMidFixedRows && 8 / wn != pq::gemm_mid_waves(m, k)) return;
     int64_t units = 0;
     for (int i = 0; i < grp.count; ++i) units += (grp.mem[i].n / 16 + nt * wn - 1) / (nt * wn);
     const int64_t wgs = units * ((nrb + rb - 1) / rb);
     const int64_t cost = (wgs + 255) / 256 * wn * nt * (34 + 8 * rb);
-    if (best.rb == 0 || cost < best_cost) {
-      best = {rb, nt, 8 / wn, wn};
-      best_cost = cost;
-    }
+    if (best.rb == 0 || cost < best.cost) best = {rb, nt, 8 / wn, wn, cost};
   };
   for (int wn = 4; wn >= 1; wn >>= 1) {
     if (m > pq::kMidFixedRows && wn < 4) consider(3, 4, wn);
@@ -48,7 +45,7 @@ MidCfg choose_mid(const pq::GemmGroup& grp, int m) {
 
 template <bool PARTIALS>
 void launch_mid(const pq::GemmGroup& grp, int bias_dtype, int y_dtype, int m, int k, hipStream_t s) {
-  const MidCfg c = choose_mid(grp, m);
+  const MidCfg c = choose_mid(grp, m, k);
   // weights that one row tile reads once are loaded non-temporally (N = 24576, M = 48: 20.5 -> 19.9 us)
   const bool once = (m + 15) / 16 <= c.rb;
 #define PQ_MID(RB_, NT_, WK_, WN_)                                                                             \
@@ -82,25 +79,26 @@ __global__ __launch_bounds__(256) void untile_a_kernel(const int8_t* __restrict_
 
 namespace pq {
 
-// From 17 rows (below, the decode kernel's one row block streams the weights
-// as fast on row-major A) to kMidMaxRows, with at least 8 groups of K, one per
-// wave.  Past 2.8 M outputs, 11 K per CU, the LDS tiles of the prefill kernel,
-// which share each operand over a workgroup, win where 128 x 256 tiles fill
-// half of the CUs, and past 3.2 M outputs its 128 x 128 tiles (N = 24576: M = 96 30.9 against 35.3 us, M = 128 35.2
-// against 32.4, M = 200 53 against 42; N = 4096, K = 4096: M = 512 20.4
-// against 24.6, M = 800 33 against 31).
+// 17 to 64 rows (else the decode kernel's row blocks on row-major codes): from 16 groups of K on, and past 32 rows
+// from 12, or from 8 for up to 16384 columns.  On fewer the final sum over the waves costs more than the order of the
+// codes saves (us with the rotation, weights from HBM, decode kernel / here: M = 24, N = 12288 K = 1024 8.8 / 11.3, K =
+// 1536 9.9 / 11.8, K = 2048 13.4 / 13.1; M = 64, N = 24576 K = 1024 17.3 / 19.6, K = 2048 25.7 / 23.4).
+//
+// Past 64 rows whichever of the mid-size GEMM (0.001 us per unit of cost and group of K) and the prefill tiles in its
+// order is estimated faster: with few column units the former leaves CUs idle in its last round, with many the
+// latter's LDS tiles share each operand over a workgroup (us with the rotation, K = 4096, two members, mid-size / in
+// chains / launch_gemm_group's prefill: M = 112 N = 12288 46.8 / 39.1 / 37.2, N = 8192 34.4 / 29.0 / 30.6; M = 144 N =
+// 8192 42.0 / 45.7 / 51.5; M = 224 N = 8192 59.0 / 47.4 / 51.7, N = 12288 81.6 / 58.1 / 54.4).
 MidGemm gemm_mid_choice(const GemmGroup& grp, int64_t m, int64_t k) {
-  if (m <= 16 || m > kMidMaxRows || k < 1024) return MidGemm::kNone;
-  int64_t n = 0, tiles256 = 0;
-  for (int i = 0; i < grp.count; ++i) {
-    n += grp.mem[i].n;
-    tiles256 += (grp.mem[i].n + 255) / 256;
-  }
-  const int64_t outputs = (m + 15) / 16 * 16 * n;
-  if (gemm_mid_waves(m) == kMidChains && m > kMidFixedRows && outputs > 2800000 &&
-      ((m + 127) / 128 * tiles256 >= 128 || outputs > 3200000))
-    return MidGemm::kChains;
-  return MidGemm::kTiled;
+  if (m <= 16 || k < 1024) return MidGemm::kNone;
+  int64_t n = 0;
+  for (int i = 0; i < grp.count; ++i) n += grp.mem[i].n;
+  if (m <= kMidFixedRows)
+    return k >= 2048 || (m > 32 && (k >= 1536 || n <= 16384)) ? MidGemm::kTiled : MidGemm::kNone;
+  const int waves = gemm_mid_waves(m, k);
+  if (waves != kMidChains) return waves != 0 ? MidGemm::kTiled : MidGemm::kNone;
+  const int64_t cost = choose_mid(grp, static_cast<int>(m), static_cast<int>(k)).cost * (k / 128);
+  return 0.001 * static_cast<double>(cost) <= gemm_chains_us(grp, m, k) ? MidGemm::kTiled : MidGemm::kChains;
 }
 
 void launch_gemm_mid(const GemmGroup& grp, int bias_dtype, int y_dtype, int m, int k, hipStream_t stream) {

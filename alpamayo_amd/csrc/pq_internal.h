@@ -150,12 +150,25 @@ PQ_HIDDEN void launch_gemm_group_partials(GemmGroup grp, int aq, int m, int k, h
 //
 // From kMidFixedRows + 1 rows on, a row's outputs must not depend on which linears share its launch (a group
 // returns the bits its members return when called one by one), so there the order of the sum over K is fixed by m
-// (gemm_mid_waves: the waves of the mid-size GEMM that split K).  The prefill tiles can take the place of its
-// kMidChains waves, not of eight, which are for few rows.
+// and k (gemm_mid_waves: the waves of the mid-size GEMM that split K, or 0: the one chain of launch_gemm_group).
+// The prefill tiles can take the place of the mid-size GEMM's kMidChains waves, not of eight, which are for few rows.
+//
+// Up to 96 rows eight waves leave fewer CUs idle (on fewer than 16 groups of K their final sum costs more than that).
+// Past 256 rows a wide launch is best on 192 x 256 tiles, which have no room for chains (gate and up, N = 24576, K =
+// 4096, M = 320: 72 us in one chain, 81 to 103 in four), so only short rows (small hidden sizes: few columns too; to
+// 384 rows) and long ones (down: N = 4096, K = 12288, M = 320: 71 us on the prefill tiles, 51 here) stay.
+// Two decoder layers in us, all sizes in one chain / by this rule, hidden 1536 / MLP 3840 M = 300 175 / 148, 4096 /
+// 12288 M = 300 474 / 422 (four chains for every K: 469).
 constexpr int kMidFixedRows = 64, kMidMaxRows = 512, kMidChains = 4;
-constexpr int gemm_mid_waves(int64_t m) { return m <= 128 ? 8 : kMidChains; }
+constexpr int gemm_mid_waves(int64_t m, int64_t k) {
+  if (k < 1024 || m > (k >= 6144 ? kMidMaxRows : k <= 3072 ? 384 : 256)) return 0;
+  return m <= 96 && k >= 2048 ? 8 : kMidChains;
+}
 enum class MidGemm { kNone, kTiled, kChains };
 PQ_HIDDEN MidGemm gemm_mid_choice(const GemmGroup& grp, int64_t m, int64_t k);
+// Time (us) of launch_gemm_chains less the fixed part of the mid-size GEMM's, fitted to launches of 65 to 512 rows
+// at K = 1024 to 12288.
+PQ_HIDDEN double gemm_chains_us(const GemmGroup& grp, int64_t m, int64_t k);
 PQ_HIDDEN void launch_gemm_chains(const GemmGroup& grp, int bias_dtype, int y_dtype, int m, int k, hipStream_t stream);
 PQ_HIDDEN void launch_gemm_chains_partials(const GemmGroup& grp, int m, int k, hipStream_t stream);
 PQ_HIDDEN void launch_gemm_mid(const GemmGroup& grp, int bias_dtype, int y_dtype, int m, int k, hipStream_t stream);

@@ -13,7 +13,7 @@ import pytest
 import torch
 
 import alpamayo_amd  # noqa: F401
-from alpamayo_amd import workloads
+from alpamayo_amd import ops, workloads
 from tests.gpu_util import gemm_instances, to_np
 from tests.test_gpu_group import _members
 from tests.test_gpu_intermediates import _check, _run
@@ -34,11 +34,20 @@ pytestmark = pytest.mark.gpu
     (200, 4224, (4096,), (True, True)),          # 33 groups: uneven K splits
     (255, 1024, (5120,), (True, True)),
     (511, 1024, (1040,), (True, True)),          # the most rows it takes, less one
-    (160, 1152, (12288, 12304), (True, True)),   # too wide: the prefill tiles in four chains of K
+    (160, 1152, (12288, 12304), (True, True)),   # too wide: 128 x 256 prefill tiles in four chains of K
     (113, 1408, (24576,), (True, True)),         # one wide member: the widest launch of the tiled kernel itself
     (96, 1152, (16384, 16400), (True, True)),    # a group too wide for one round, each member in less than one
     (113, 1408, (8192,) * 4, (True, True)),
-    (500, 1152, (6144, 1280), (True, True)),     # 128 x 128 tiles in four chains
+    (500, 1152, (6144, 1280), (True, True)),     # short rows past 384 rows: the prefill tiles in one chain
+    (96, 2048, (12288, 48), (True, True)),       # the most rows on eight waves
+    (97, 2048, (8192, 8208), (True, True)),      # and the first past them: 64 x 128 tiles in four chains
+    (128, 1024, (12288, 4112), (True, True)),
+    (256, 4096, (4096, 1040, 1024), (True, True)),
+    (257, 3072, (3072, 3088), (True, True)),     # short rows up to 384 rows
+    (384, 1024, (5120, 272), (True, True)),
+    (320, 6144, (16384, 1040), (True, True)),    # long rows up to 512: 128 x 256 tiles in four chains
+    (512, 6144, (4096, 48), (False, True)),
+    (513, 6144, (4096, 48), (True, True)),       # the first row count past the mid-size GEMM
 ])
 def test_tiled_gemm(M, K, ns, flags):
     print(f"tiled GEMM M={M} K={K} ns={ns} flags={flags}", flush=True)
@@ -86,3 +95,33 @@ def test_parity_form_runs_the_tiles_of_the_product(M, K, ns):
                  (lambda: _run(mbs, x, 8, (True, True)),
                   lambda: torch.ops.paroquant.w4a8_linear_group(x, *args, torch.bfloat16)))
     assert want and got == want
+
+
+SKINNY, MID, PREFILL = "gemm_skinny", "gemm_mid", "gemm_prefill"
+
+
+@pytest.mark.parametrize("M,K,ns,kernel,rows", [
+    (16, 4096, (4096,), SKINNY, None), (17, 4096, (4096,), MID, None),
+    (24, 1024, (12288,), SKINNY, None), (24, 1536, (4096,), SKINNY, None), (24, 2048, (4096,), MID, None),
+    (33, 1024, (4096,), MID, None), (33, 1024, (24576,), SKINNY, None), (33, 1536, (24576,), MID, None),
+    (64, 4096, (12288, 12288), MID, None), (65, 4096, (12288, 12288), MID, None),
+    (112, 4096, (12288, 12288), PREFILL, 64), (112, 4096, (4096, 1024, 1024), MID, None),
+    (144, 4096, (8192, 8192), MID, None), (200, 4096, (12288, 12288), PREFILL, 128), (256, 4096, (4096,), MID, None),
+    (257, 4096, (4096,), PREFILL, None), (320, 4096, (12288, 12288), PREFILL, 192),
+    (384, 4096, (12288, 12288), PREFILL, 192), (320, 12288, (4096,), MID, None), (500, 1024, (4096,), PREFILL, None),
+    (300, 2048, (2048, 512, 512), MID, None), (400, 2048, (2048, 512, 512), PREFILL, None),
+    (512, 12288, (4096,), MID, None), (513, 12288, (4096,), PREFILL, None),
+])
+def test_kernel_by_size(M, K, ns, kernel, rows):
+    """The kernel, and of gemm_prefill the rows of a tile, that each range of sizes measured fastest on."""
+    print(f"dispatch M={M} K={K} ns={ns}", flush=True)
+    dev = "cuda"
+    identity = torch.stack([torch.ones(1, K // 2), torch.zeros(1, K // 2)], dim=-1)
+    rot_idx, rot_cs = (t.to(dev) for t in ops.pack_rotation(torch.arange(128).repeat(1, K // 128), identity))
+    wps = [torch.zeros(n // 16, K // 128, 64, 16, dtype=torch.uint8, device=dev) for n in ns]
+    wms = [torch.zeros(n // 16, K // 128, 16, dtype=torch.int32, device=dev) for n in ns]
+    c = len(ns)
+    x = torch.zeros(M, K, dtype=torch.bfloat16, device=dev)
+    found = gemm_instances(lambda: torch.ops.paroquant.w4a8_linear_group(
+        x, [rot_idx] * c, [rot_cs] * c, [None] * c, 1, wps, wms, [None] * c, True, True, torch.bfloat16))
+    assert [f[0] for f in found] == [kernel] and (rows is None or found[0][1][0] == str(rows))
