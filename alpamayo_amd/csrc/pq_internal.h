@@ -50,12 +50,12 @@ struct RotMember {
   void* out;
   float* out_scale;
   void* xrot;
+  int tiled;   // row kernel: rows m of the tiled order (pqd::a_tile_offset, a16_tile_offset) of the int8 codes
+               // and of the fp16 rows; 0: row-major
 };
 struct RotGroup {
   RotMember mem[kMaxGroup];
   int count;
-  int tiled;   // row kernel: rows m of the tiled order (pqd::a_tile_offset, a16_tile_offset) of the int8 codes
-               // and of the fp16 rows; 0: row-major
 };
 
 // Per-token int8 quantization of a split rotation's output (launch_quant_split):

@@ -194,7 +194,8 @@ int linear_group(const char* who, const void* x, int x_dtype, const pq_linear_me
   // The mid-size GEMM reads the int8 codes in the tiled order, which the quant launches then write.
   const pq::MidGemm mid = path != Path::kSplit ? pq::gemm_mid_choice(gg, m, k) : pq::MidGemm::kNone;
   const bool tiled = mid == pq::MidGemm::kTiled;
-  rg.tiled = qg.tiled = tiled ? M : 0;
+  qg.tiled = tiled ? M : 0;
+  for (int i = 0; i < count; ++i) rg.mem[i].tiled = qg.tiled;
   int st = PQ_OK;
   if (stage == 2) {
     // the GEMM alone, from the workspace stage 1 filled

@@ -68,6 +68,7 @@ __global__ __launch_bounds__(kRQWaves * 64) void rotate_quant_kernel(const void*
   int8_t* __restrict__ xq = static_cast<int8_t*>(mb.out);
   float* __restrict__ xscale = mb.out_scale;
   uint16_t* __restrict__ xrot = static_cast<uint16_t*>(mb.xrot);
+  const int tiled = mb.tiled;
   extern __shared__ __attribute__((aligned(16))) unsigned char lds_raw[];
   __shared__ float red[kRQWaves][RB];
   using RowT = typename std::conditional<MAT16, uint16_t, float>::type;
@@ -369,7 +370,7 @@ __global__ __launch_bounds__(kRQWaves * 64) void rotate_quant_kernel(const void*
           uint32_t w[4];
 #pragma unroll
           for (int m = 0; m < 4; ++m) w[m] = pqd::f16_pair(d, 2 * m * RB + r, (2 * m + 1) * RB + r);
-          *reinterpret_cast<uint4*>(xrot + (grp.tiled ? pqd::a16_tile_offset(row0 + r, c8, grp.tiled, G) : ro)) =
+          *reinterpret_cast<uint4*>(xrot + (tiled ? pqd::a16_tile_offset(row0 + r, c8, tiled, G) : ro)) =
               make_uint4(w[0], w[1], w[2], w[3]);
         }
         if (xq != nullptr) {
@@ -380,7 +381,7 @@ __global__ __launch_bounds__(kRQWaves * 64) void rotate_quant_kernel(const void*
             const int i = k * RB + r;
             c[k] = pqd::quant_scaled(pqd::mul_f16(d[i >> 1], (i & 1) != 0, inv));
           }
-          *reinterpret_cast<uint2*>(xq + (grp.tiled ? pqd::a_tile_offset(row0 + r, c8, grp.tiled, G) : ro)) =
+          *reinterpret_cast<uint2*>(xq + (tiled ? pqd::a_tile_offset(row0 + r, c8, tiled, G) : ro)) =
               make_uint2(pqd::pack4(c[0], c[1], c[2], c[3]), pqd::pack4(c[4], c[5], c[6], c[7]));
         }
       }
@@ -403,14 +404,14 @@ __global__ __launch_bounds__(kRQWaves * 64) void rotate_quant_kernel(const void*
         o.y = pqd::pk_f16(f[2], f[3]);
         o.z = pqd::pk_f16(f[4], f[5]);
         o.w = pqd::pk_f16(f[6], f[7]);
-        *reinterpret_cast<uint4*>(xrot + (grp.tiled ? pqd::a16_tile_offset(row0 + r, c8, grp.tiled, G)
+        *reinterpret_cast<uint4*>(xrot + (tiled ? pqd::a16_tile_offset(row0 + r, c8, tiled, G)
                                                     : (row0 + r) * h + c8)) = o;
       }
       if (xq != nullptr) {
         uint2 o;
         o.x = quant4(f[0], f[1], f[2], f[3], inv);
         o.y = quant4(f[4], f[5], f[6], f[7], inv);
-        *reinterpret_cast<uint2*>(xq + (grp.tiled ? pqd::a_tile_offset(row0 + r, c8, grp.tiled, G) : (row0 + r) * h + c8)) = o;
+        *reinterpret_cast<uint2*>(xq + (tiled ? pqd::a_tile_offset(row0 + r, c8, tiled, G) : (row0 + r) * h + c8)) = o;
       }
     }
   }

@@ -54,9 +54,12 @@ struct W16Group {
   int count;
 };
 
-// Mid-size GEMM on tiled fp16 rows (pqd::a16_tile_offset): whether m rows of the group run it, and its launch
+// Mid-size GEMM on tiled fp16 rows (pqd::a16_tile_offset): whether m rows of a linear of n columns run it, alone or in
+// a group (the prefill tiles sum in another order, so the choice looks at the member alone), and its launch
 // (pq_w4a16_mid.hip).
-PQ_HIDDEN bool w16_mid_takes(const W16Group& grp, int64_t m, int64_t k);
+PQ_HIDDEN bool w16_mid_takes(int64_t m, int64_t n, int64_t k);
+// Time (us) of the prefill tiles for m > 16 rows, less the fixed part of a launch of the mid-size GEMM.
+PQ_HIDDEN double w16_prefill_us(int64_t m, int64_t n, int64_t k);
 PQ_HIDDEN void launch_w16_mid(const W16Group& grp, int bias_dtype, int y_dtype, int m, int k, hipStream_t stream);
 
 }  // namespace pqw16

@@ -341,29 +341,39 @@ void launch_w16_prefill_t(const W16Args& ar, int bias_dtype, int y_dtype, int M,
   w16_prefill<BM, BN, WM, WN><<<grid, WM * WN * 64, kW16Stages * STAGE, stream>>>(ar, bias_dtype, y_dtype, M, K);
 }
 
-// 32 x 128 tiles when one round of them covers the output (below); else the
-// cheapest of 192 x 256, 128 x 256 (8 waves of 192 or 128 rows x 32
-// columns) and 128 x 128 tiles (4 waves) by the measured cost of their
+// 32 x 128 tiles when one round of them covers the output (17-256 tokens at
+// N = 4096): each workgroup walks all of K, so its time follows its rows (M =
+// 64-256: 42 -> 26 us at K = 4096, M = 128: 115 -> 71 us at K = 12288 against 128
+// x 128); else the cheapest of 192 x 256, 128 x 256 (8 waves of 192 or 128 rows
+// x 32 columns) and 128 x 128 tiles (4 waves) by the measured cost of their
 // rounds of 256 workgroups (one per CU), in units of a full round of
 // 192 x 256 tiles (K = 4096): a full round of 128 x 256 tiles takes 0.74 of
 // it and one of 128 x 128 tiles 0.45; a last, partly filled round costs 0.77
 // of a full one on 192 x 256 tiles and 0.9 on the smaller ones.  M = 4096,
 // N = 4096: 171 -> 144 us (128 x 256); M = 1024, N = 4096: 46 us on 128 x 128
 // against 57 us on 128 x 256.
-void launch_w16_prefill(const W16Args& ar, int bias_dtype, int y_dtype, int M, int K, hipStream_t stream) {
+struct W16Tiles {
+  int bm, bn;
+  double rounds;   // their cost
+};
+W16Tiles choose_w16_prefill(int64_t m, int64_t n) {
   auto rounds = [](int64_t tiles, double full, double partial) {
     return full * static_cast<double>(tiles / 256) + (tiles % 256 != 0 ? full * partial : 0.0);
   };
-  const double big = rounds(static_cast<int64_t>((M + 191) / 192) * ((ar.n + 255) / 256), 1.0, 0.77);
-  const double mid = rounds(static_cast<int64_t>((M + 127) / 128) * ((ar.n + 255) / 256), 0.74, 0.9);
-  const double small = rounds(static_cast<int64_t>((M + 127) / 128) * ((ar.n + 127) / 128), 0.45, 0.9);
-  if (big <= mid && big <= small) launch_w16_prefill_t<192, 256, 1, 8>(ar, bias_dtype, y_dtype, M, K, stream);
-  else if (mid <= small) launch_w16_prefill_t<128, 256, 1, 8>(ar, bias_dtype, y_dtype, M, K, stream);
-  // at most one round of 32-row tiles (17-256 tokens at N = 4096): each
-  // workgroup walks all of K, so its time follows its rows (M = 64-256: 42
-  // -> 26 us at K = 4096, M = 128: 115 -> 71 us at K = 12288 against 128 x 128)
-  else if (static_cast<int64_t>((M + 31) / 32) * ((ar.n + 127) / 128) <= 256)
-    launch_w16_prefill_t<32, 128, 1, 4>(ar, bias_dtype, y_dtype, M, K, stream);
+  const double big = rounds((m + 191) / 192 * ((n + 255) / 256), 1.0, 0.77);
+  const double mid = rounds((m + 127) / 128 * ((n + 255) / 256), 0.74, 0.9);
+  const double small = rounds((m + 127) / 128 * ((n + 127) / 128), 0.45, 0.9);
+  if (big <= mid && big <= small) return {192, 256, big};
+  if (mid <= small) return {128, 256, mid};
+  if ((m + 31) / 32 * ((n + 127) / 128) <= 256) return {32, 128, 0.0};
+  return {128, 128, small};
+}
+
+void launch_w16_prefill(const W16Args& ar, int bias_dtype, int y_dtype, int M, int K, hipStream_t stream) {
+  const W16Tiles t = choose_w16_prefill(M, ar.n);
+  if (t.bm == 192) launch_w16_prefill_t<192, 256, 1, 8>(ar, bias_dtype, y_dtype, M, K, stream);
+  else if (t.bn == 256) launch_w16_prefill_t<128, 256, 1, 8>(ar, bias_dtype, y_dtype, M, K, stream);
+  else if (t.bm == 32) launch_w16_prefill_t<32, 128, 1, 4>(ar, bias_dtype, y_dtype, M, K, stream);
   else launch_w16_prefill_t<128, 128, 1, 4>(ar, bias_dtype, y_dtype, M, K, stream);
 }
 
@@ -478,6 +488,14 @@ size_t w16_linear_workspace(int64_t m, int64_t k) {
 
 }  // namespace
 
+double pqw16::w16_prefill_us(int64_t m, int64_t n, int64_t k) {
+  const W16Tiles t = choose_w16_prefill(m, n);
+  const double g = static_cast<double>(k / 128);
+  if (t.bm == 32) return 0.64 * g + 0.5;
+  if (t.bn == 128) return (0.71 * t.rounds + 0.76) * g + 4.0;
+  return (t.bm == 192 ? 2.0 * t.rounds : 1.72 - 0.21 * t.rounds) * g + 4.0;
+}
+
 extern "C" int pq_w4a16_gemm(const void* x, const uint8_t* wpack, const uint32_t* wmeta, const void* bias,
                              int bias_dtype, void* y, int y_dtype, int64_t m, int64_t n, int64_t k, int group_size,
                              void* stream) {
@@ -552,16 +570,22 @@ int w16_linear_group(const char* who, const void* x, int x_dtype, const pq_linea
     gg.mem[i] = {reinterpret_cast<const uint16_t*>(rows), mb.wpack, mb.wmeta, mb.bias, mb.y, static_cast<int>(mb.n)};
   }
   const unsigned rflags = flags | PQ_RQ_MATERIALIZE_FP16;
+  // The members on the mid-size GEMM, in one launch, read their fp16 rows in the tiled order, which the row kernel
+  // then writes; the others run as ever.
+  W16Group mid{}, rest{};
+  for (int i = 0; i < count; ++i) {
+    const bool tiled = !split && w16_mid_takes(m, members[i].n, k);
+    rg.mem[i].tiled = tiled ? M : 0;
+    W16Group& g = tiled ? mid : rest;
+    g.mem[g.count++] = gg.mem[i];
+  }
   // One row per wave, as the W4A8 linear's split rotation.
-  // The mid-size GEMM reads the fp16 rows in the tiled order, which the row kernel then writes.
-  const bool mid = !split && w16_mid_takes(gg, m, k);
-  rg.tiled = mid ? M : 0;
   if (split) pq::launch_rotate_split(x, x_dtype, rg, M, K, krot, rflags, s, norm, 1);
   else pq::launch_rotate_quant_group(x, x_dtype, rg, m, K, krot, rflags, s, norm);
   int st = pq::launch_status("W4A16 linear rotation launch");
   if (st != PQ_OK) return st;
-  if (mid) launch_w16_mid(gg, bias_dtype, y_dtype, M, K, s);
-  else launch_w16_gemm_group(gg, bias_dtype, y_dtype, M, K, s);
+  if (mid.count > 0) launch_w16_mid(mid, bias_dtype, y_dtype, M, K, s);
+  if (rest.count > 0) launch_w16_gemm_group(rest, bias_dtype, y_dtype, M, K, s);
   return pq::launch_status("W4A16 linear GEMM launch");
 }
 

@@ -1,10 +1,15 @@
 // W4A16 GEMM for 17 to a few hundred rows, on tiled fp16 activations: the
 // structure of the W4A8 one (pq_gemm_mid.h) -- a wave owns RB x NT blocks of
-// 16 x 16 outputs and every WK-th group of K, operands straight into registers
+// 16 x 16 outputs and one of WK parts of K, operands straight into registers
 // two groups ahead, no barrier before the final LDS sum -- with the weights
 // dequantized once per wave and block and v_mfma_f32_16x16x32_f16 summing over
-// all of a wave's groups (no scaling per group).  The dequantization, 56 VALU
+// the groups (no scaling per group).  The dequantization, 56 VALU
 // instructions per 16 columns and group, is what RB rows blocks share.
+//
+// A row's outputs are the same bits in every configuration, so that a group of
+// linears returns what its members return alone: K falls into kParts16 parts,
+// a wave walks one of them or two neighbours, every part's sum starts from zero
+// and goes to LDS, and there the parts are added in one order.
 #pragma once
 
 #include "pq_gemm_mid.h"
@@ -14,6 +19,11 @@ namespace pqmid {
 
 using namespace pqw16;
 
+constexpr int kParts16 = 8;
+
+template <int RB, int NT, int WN>
+constexpr size_t lds_bytes16() { return static_cast<size_t>(kParts16) * WN * RB * NT * 4 * 64 * sizeof(float); }
+
 template <int RB, int NT>
 struct Stage16 {
   v8h a[RB][4];
@@ -21,8 +31,9 @@ struct Stage16 {
   uint32_t meta[NT];
 };
 
+// (bounds of the 4-wave instance: three workgroups per CU)
 template <int RB, int NT, int WK, int WN>
-__global__ __launch_bounds__(WK * WN * 64) void w16_mid(const W16Group grp, int bias_dtype, int y_dtype, int M, int K) {
+__global__ __launch_bounds__(WK * WN * 64, WK * WN == 4 ? 3 : 2) void w16_mid(const W16Group grp, int bias_dtype, int y_dtype, int M, int K) {
   extern __shared__ __attribute__((aligned(16))) float red[];
   const int G = K >> 7;
   const int nrb = (M + 15) >> 4;
@@ -77,10 +88,6 @@ __global__ __launch_bounds__(WK * WN * 64) void w16_mid(const W16Group grp, int 
   };
 
   v4f acc[RB][NT];
-#pragma unroll
-  for (int b = 0; b < RB; ++b)
-#pragma unroll
-    for (int nt = 0; nt < NT; ++nt) acc[b][nt] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
   auto compute = [&](const Stage16<RB, NT>& s) {
 #pragma unroll
     for (int nt = 0; nt < NT; ++nt) {
@@ -94,33 +101,10 @@ __global__ __launch_bounds__(WK * WN * 64) void w16_mid(const W16Group grp, int 
     }
   };
 
-  // Two register stages, the tail peeled so that no load sits behind a branch.
-  const int n = (G - wk + WK - 1) / WK;
-  auto grp_of = [&](int i) { return wk + i * WK; };
-  Stage16<RB, NT> s0, s1;
-  load(s0, grp_of(0));
-  load(s1, grp_of(min(1, n - 1)));
-  int i = 0;
-  for (; i + 3 < n; i += 2) {
-    compute(s0);
-    load(s0, grp_of(i + 2));
-    compute(s1);
-    load(s1, grp_of(i + 3));
-  }
-  if (n - i == 3) {
-    compute(s0);
-    load(s0, grp_of(i + 2));
-    compute(s1);
-    compute(s0);
-  } else {
-    compute(s0);
-    if (n - i == 2) compute(s1);
-  }
-
-  constexpr int KK = kept(WK);
+  // The sums of parts: red[part][wn][(b, nt, v)][lane]
   constexpr int REGS = RB * NT * 4;
-  auto slot = [&](int k) { return red + static_cast<size_t>(k * WN + wn) * REGS * 64 + lane; };
-  auto put = [&](float* dst) {
+  auto put = [&](int part) {
+    float* dst = red + static_cast<size_t>(part * WN + wn) * REGS * 64 + lane;
 #pragma unroll
     for (int b = 0; b < RB; ++b)
 #pragma unroll
@@ -128,21 +112,19 @@ __global__ __launch_bounds__(WK * WN * 64) void w16_mid(const W16Group grp, int 
 #pragma unroll
         for (int v = 0; v < 4; ++v) dst[((b * NT + nt) * 4 + v) * 64] = acc[b][nt][v];
   };
-  if constexpr (KK < WK) {
-    if (wk >= KK) put(slot(wk - KK));
-    __syncthreads();
-    if (wk < KK) {
-      const float* src = slot(wk);
+  // Wave wk walks parts wk PW .. wk PW + PW - 1, one after the other (the host keeps kParts16 <= G).  One loop over
+  // both, with the sum put away in its middle, costs the 4-wave instance its third wave per SIMD.
+  constexpr int PW = kParts16 / WK;
+#pragma unroll 1
+  for (int part = wk * PW; part < (wk + 1) * PW; ++part) {
+    const int gb = part * G / kParts16;
 #pragma unroll
-      for (int b = 0; b < RB; ++b)
+    for (int b = 0; b < RB; ++b)
 #pragma unroll
-        for (int nt = 0; nt < NT; ++nt)
-#pragma unroll
-          for (int v = 0; v < 4; ++v) acc[b][nt][v] = acc[b][nt][v] + src[((b * NT + nt) * 4 + v) * 64];
-      put(slot(wk));   // the wave overwrites only what it has just read
-    }
-  } else {
-    put(slot(wk));
+      for (int nt = 0; nt < NT; ++nt) acc[b][nt] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
+    walk<Stage16<RB, NT>>((part + 1) * G / kParts16 - gb, [&](Stage16<RB, NT>& s, int i) { load(s, gb + i); },
+                          [&](const Stage16<RB, NT>& s, int) { compute(s); });
+    put(part);
   }
   __syncthreads();
   constexpr int CH = 4 * NT * WN;   // 4-column chunks per row
@@ -154,22 +136,20 @@ __global__ __launch_bounds__(WK * WN * 64) void w16_mid(const W16Group grp, int 
     if (m >= M || tile >= ntiles) continue;
     const int b = row >> 4, jj = (row >> 2) & 3, v = row & 3;
     const float* src = red + (static_cast<size_t>(wc) * REGS + (b * NT + nt) * 4 + v) * 64 + jj * 16 + cq * 4;
-    float f[4];
-    {
-      const float4 s = *reinterpret_cast<const float4*>(src);
-      f[0] = s.x;
-      f[1] = s.y;
-      f[2] = s.z;
-      f[3] = s.w;
-    }
+    float4 p[kParts16];
 #pragma unroll
-    for (int k = 1; k < KK; ++k) {
-      const float4 o = *reinterpret_cast<const float4*>(src + static_cast<size_t>(k) * WN * REGS * 64);
-      f[0] += o.x;
-      f[1] += o.y;
-      f[2] += o.z;
-      f[3] += o.w;
-    }
+    for (int k = 0; k < kParts16; ++k)
+      p[k] = *reinterpret_cast<const float4*>(src + static_cast<size_t>(k) * WN * REGS * 64);
+#pragma unroll
+    for (int d = 1; d < kParts16; d *= 2)   // neighbours first
+#pragma unroll
+      for (int k = 0; k < kParts16; k += 2 * d) {
+        p[k].x += p[k + d].x;
+        p[k].y += p[k + d].y;
+        p[k].z += p[k + d].z;
+        p[k].w += p[k + d].w;
+      }
+    float f[4] = {p[0].x, p[0].y, p[0].z, p[0].w};
     const int col = tile * 16 + cq * 4;
     if (mb.bias != nullptr) {
 #pragma unroll
@@ -194,7 +174,7 @@ void launch_w16_mid_t(W16Group grp, int bias_dtype, int y_dtype, int M, int K, h
   for (int i = 0; i < grp.count; ++i) grp.first[i + 1] = grp.first[i] + (grp.mem[i].n / 16 + NT * WN - 1) / (NT * WN);
   const int nrt = ((M + 15) / 16 + RB - 1) / RB;
   const unsigned grid = static_cast<unsigned>(grp.first[grp.count]) * static_cast<unsigned>(nrt);
-  w16_mid<RB, NT, WK, WN><<<grid, WK * WN * 64, lds_bytes<RB, NT, WK, WN>(), stream>>>(grp, bias_dtype, y_dtype, M, K);
+  w16_mid<RB, NT, WK, WN><<<grid, WK * WN * 64, lds_bytes16<RB, NT, WN>(), stream>>>(grp, bias_dtype, y_dtype, M, K);
 }
 
 }  // namespace pqmid

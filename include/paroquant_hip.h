@@ -360,9 +360,12 @@ int pq_w4a16_linear(const void* x, int x_dtype, const uint32_t* rot_idx, const f
 size_t pq_w4a16_linear_group_workspace_size(int64_t m, int64_t k, int count);
 
 /* pq_w4a16_linear for count (1..4) linears that read the same x (q/k/v,
- * gate/up): one rotation launch over all members and, for m <= 16 and at
- * mid sizes (up to 3.2 M outputs), one GEMM launch over their concatenated
- * columns (else one GEMM launch per member).  Each member's y is what pq_w4a16_linear gives for it.  Members
+ * gate/up): one rotation launch over all members, then, for m <= 16, one GEMM
+ * launch over their concatenated columns; for larger m one launch of the
+ * mid-size GEMM over the members it takes (17 to 512 rows, by the size of each
+ * member) and one of the prefill GEMM per other member.  Each member's y is
+ * what pq_w4a16_linear gives for it, bit for bit for m > 16 (for m <= 16 the
+ * float32 sum over K may be split over another number of waves).  Members
  * as for pq_w4a8_linear_group.  No counterpart in the reference (its
  * linears run one by one, rotation_linear.py:136-139 each). */
 int pq_w4a16_linear_group(const void* x, int x_dtype, const pq_linear_member* members, int count,

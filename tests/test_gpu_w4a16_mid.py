@@ -15,6 +15,15 @@ from tests.gpu_util import packed_rotation
 pytestmark = pytest.mark.gpu
 
 
+def _operands(n, K, seed, with_bias):
+    spec = workloads.linear_spec("t", n, K, workloads.generator(seed), keep_codes=True)
+    rot_idx, rot_cs, _, _ = packed_rotation(spec.pairs, spec.theta)
+    s, sz = workloads.w16_scales(spec.w)
+    wp, wm = torch.ops.paroquant.w4a16_prepack(spec.w.awq_qweight.cuda(), s.cuda(), sz.cuda())
+    b = torch.randn(n, generator=workloads.generator(n)).half().cuda() if with_bias else None
+    return (rot_idx.cuda(), rot_cs.cuda(), spec.channel_scales.float().reshape(-1).cuda(), wp, wm, b), spec, s, sz
+
+
 @pytest.mark.parametrize("M,K,ns", [
     (17, 1024, (16,)), (31, 1152, (1040,)), (33, 4096, (4096, 1024, 1024)), (48, 12288, (4096,)), (64, 1408, (12288, 12304)),
     (65, 4096, (4096,)), (97, 2048, (1040, 80)), (129, 4224, (4096,)), (200, 1024, (5120,)), (255, 1152, (4112,)),
@@ -25,13 +34,8 @@ def test_tiled_w16_gemm(M, K, ns):
     x = workloads.activations(M, K, workloads.generator(5000 + M)).half().cuda()
     ops_, refs, bounds = [], [], []
     for i, n in enumerate(ns):
-        spec = workloads.linear_spec(f"t{i}", n, K, workloads.generator(zlib.crc32(f"{K}{n}{i}".encode())),
-                                     keep_codes=True)
-        rot_idx, rot_cs, _, _ = packed_rotation(spec.pairs, spec.theta)
-        s, sz = workloads.w16_scales(spec.w)
-        wp, wm = torch.ops.paroquant.w4a16_prepack(spec.w.awq_qweight.cuda(), s.cuda(), sz.cuda())
-        b = torch.randn(n, generator=workloads.generator(n)).half().cuda() if i == 0 else None
-        o = (rot_idx.cuda(), rot_cs.cuda(), spec.channel_scales.float().reshape(-1).cuda(), wp, wm, b)
+        o, spec, s, sz = _operands(n, K, zlib.crc32(f"{K}{n}{i}".encode()), i == 0)
+        b = o[5]
         ops_.append(o)
         _, _, rows = torch.ops.paroquant.rotate_quant_i8_rot(x, o[0], o[1], o[2], 8, False, True)
         q = spec.w.codes.cuda().double().view(n, K // 128, 128)
@@ -47,3 +51,27 @@ def test_tiled_w16_gemm(M, K, ns):
     for y, yh, ref, bound in zip(ys, y16, refs, bounds):
         assert torch.all((y.double() - ref).abs() <= bound)
         assert torch.equal(yh.view(torch.int16), y.half().view(torch.int16))
+
+
+@pytest.mark.parametrize("M,K,ns", [
+    (17, 1152, (4096, 1040)),
+    (33, 1024, (12288, 12304)),          # one group per part of K, on both widths of workgroup
+    (48, 2176, (9728, 9728)),            # 17 groups: parts of two and three
+    (64, 1152, (12288, 12288)),          # a lone member this wide asks for another split of K than the pair
+    (65, 1024, (16, 8192)),
+    (96, 4096, (12288, 12288, 1024)),    # the pair asks for another number of waves than the narrow member
+    (130, 1024, (12288, 12288)),
+    (320, 2048, (4096, 1024, 1024)),
+    (500, 1152, (5120, 1280, 1280)),     # the first member runs the prefill tiles by itself
+    (512, 1408, (4096, 5120, 48, 16)),
+])
+def test_group_returns_its_members_bits(M, K, ns):
+    print(f"W4A16 group against its members M={M} K={K} ns={ns}", flush=True)
+    x = workloads.activations(M, K, workloads.generator(6000 + M)).half().cuda()
+    ops_ = [_operands(n, K, 77 + i, i % 2 == 0)[0] for i, n in enumerate(ns)]
+    get = lambda i: [o[i] for o in ops_]   # noqa: E731
+    ys = torch.ops.paroquant.w4a16_linear_group(x, get(0), get(1), get(2), 8, get(3), get(4), get(5), False,
+                                                torch.float32)
+    for o, y in zip(ops_, ys):
+        single = torch.ops.paroquant.w4a16_linear(x, *o[:3], 8, *o[3:], False, torch.float32)
+        assert torch.equal(y, single)
