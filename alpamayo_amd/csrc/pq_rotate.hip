@@ -426,8 +426,12 @@ void launch_rotate(const void* x, void* y, uint8_t* sc, const int16_t* idx, cons
 // chain serves too few rows to pay for being derived (fp16, 8 layers, tile
 // form -> chain in us: 512 x 4096 9.6 -> 10.0, 1024 x 4096 15.6 -> 12.9, 2100 x
 // 4096 27.3 -> 20.1, 1024 x 12288 37.4 -> 25.7; 16 layers 1024 x 4096 24.1 ->
-// 18.7; float32, 8 layers, 8192 x 4096 102 -> 58).
-constexpr int64_t kChainElems = 1 << 22;
+// 18.7; float32, 8 layers, 8192 x 4096 102 -> 58).  One and two layers are
+// little to save, from 6 M (1026 x 4096 8.7 -> 9.4, 1465 x 4096 11.8 -> 9.9;
+// with MXFP4 codes 11.9 -> 10.3 already).  And 32 rows at least, a step of a
+// workgroup: fewer, longer rows derive a chain per 128 channels for them (16 x
+// 262144 15.5 -> 22.3, 4 x 1048576 44 -> 72; 33 x 131072 20.1 -> 17.7).
+constexpr int64_t kChainElems = 1 << 22, kChainElemsFewLayers = 6000000, kChainRows = 32;
 
 template <int DT, bool MX>
 void launch_chain(const void* x, void* y, uint8_t* sc, const int16_t* idx, const void* theta, const void* scales,
@@ -450,7 +454,7 @@ void launch_chain(const void* x, void* y, uint8_t* sc, const int16_t* idx, const
 template <int DT>
 void launch_rotate_dt(const void* x, void* y, uint8_t* sc, const int16_t* idx, const void* theta,
                       const void* scales, int64_t rows, int h, int krot, int group, hipStream_t stream) {
-  if (rows * h >= kChainElems) {
+  if (rows >= kChainRows && rows * h >= (krot <= 2 && sc == nullptr ? kChainElemsFewLayers : kChainElems)) {
     if (sc != nullptr) launch_chain<DT, true>(x, y, sc, idx, theta, scales, rows, h, krot, group, stream);
     else launch_chain<DT, false>(x, y, sc, idx, theta, scales, rows, h, krot, group, stream);
     return;

@@ -18,7 +18,7 @@
 //
 // The angle and scale gradients are sums over all rows.  A workgroup walks
 // its column of row tiles grid-stride and keeps running sums in registers,
-// the 4 waves are summed through LDS in a fixed order, and each workgroup row
+// its waves are summed through LDS in a fixed order, and each workgroup row
 // writes one partial per angle / channel; a second kernel adds the partials
 // in a fixed order.  The result is deterministic (no atomics).
 #include <algorithm>
@@ -71,9 +71,11 @@ void launch_bwd(const void* x, const void* gy, void* gx, void* g_theta, void* g_
                 hipStream_t s) {
   // The register chain where a workgroup has rows enough to pay for deriving it (tile form -> chain, us, 8 layers:
   // 128 x 4096 11.5 -> 13.0, 256 x 4096 15.8 -> 13.2, 64 x 12288 12.2 -> 11.0, 1024 x 4096 50.7 -> 22.5, 8192 x 4096
-  // float32 221 -> 106; 16 layers 256 x 4096 17.6 -> 26.7, 512 x 4096 37.8 -> 31.5), on at most one workgroup per CU
-  // (what its registers allow); else the tile form on every workgroup row the workspace has room for.
-  const bool chain = rows * h >= (krot <= 8 ? 3 << 18 : 1 << 21);
+  // float32 221 -> 106; 16 layers 256 x 4096 17.6 -> 26.7, 512 x 4096 37.8 -> 31.5), a step of 32 of them at least (8
+  // layers 16 x 49152 12.2 -> 17.3, 1 x 1048576 95 -> 222, 34 x 65536 25.2 -> 22.9; 16 layers 34 x 65536 47 -> 51, 49 x
+  // 65536 63 -> 54), on at most one workgroup per CU (what its registers allow); else the tile form on every workgroup
+  // row the workspace has room for.
+  const bool chain = krot <= 8 ? rows >= 32 && rows * h >= 3 << 18 : rows >= 48 && rows * h >= 1 << 21;
   const int64_t chunks = (h + 127) / 128;
   const int nb = static_cast<int>(
       chain ? std::min<int64_t>(bwd_blocks(rows), std::max<int64_t>(1, 256 / chunks)) : bwd_blocks(rows));

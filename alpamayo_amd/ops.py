@@ -184,17 +184,22 @@ def _rotate_args(x, idx_ij, theta, scales):
 
 
 # Packed operands of rotation::rotate's (pairs, angles, scales), registered by whoever derived them
-# (Rotation.prepare()): from 1024 rows up to _PACKED_MAX_ELEMS the register-chain kernel of the fused linear runs
-# whole rows faster than the kernel that derives the chain from the raw operands, which past that size takes 128
-# channels of many rows per workgroup and wins (bfloat16 to MXFP4, us: 3072 x 1024 10.5 against 13.1, 1024 x 4096 13.7 /
-# 13.4, 2100 x 4096 26.6 / 21.3, 3072 x 4096 28.0 / 24.9, 1024 x 12288 34.8 / 27.4).  The results are the same (cos/sin
-# of each angle in float64, rounded once).  The op itself only looks them up -- it never packs, copies to the host or
-# synchronizes -- and runs the tile kernel, which derives its parameters on the device, when nothing
-# current is registered for its exact tensors.
+# (Rotation.prepare()): from 1024 rows up to _packed_max_elems() the register-chain kernel of the fused linear runs
+# whole rows faster than the kernels that work from the raw operands, which past that size take 128 channels of many
+# rows per workgroup, derive their chain on the device and win (bfloat16 to MXFP4, us: 3072 x 1024 10.5 against 13.1,
+# 1024 x 4096 13.7 / 13.4, 2100 x 4096 26.6 / 21.3, 3072 x 4096 28.0 / 24.9, 1024 x 12288 34.8 / 27.4; plain rows of 8
+# layers 1024 x 4096 12.5 / 13.7, 1465 x 4096 20.8 / 17.0, of 4 layers 2051 x 2048 0.91 of the time).  The results are
+# the same (cos/sin of each angle in float64, rounded once).  The op itself only looks them up -- it never packs,
+# copies to the host or synchronizes -- and works from the raw operands when nothing current is registered for its
+# exact tensors.
 _PACK_REGISTRY: "OrderedDict" = OrderedDict()
 _PACK_REGISTRY_MAX = 4096
 _PACKED_MIN_ROWS = 1024
-_PACKED_MAX_ELEMS = 1 << 22
+
+
+def _packed_max_elems(krot: int, mxfp4: bool) -> int:
+    return 5 << 20 if krot == 8 and not mxfp4 else 1 << 22
+
 
 
 def _none_ref():
@@ -267,7 +272,7 @@ def _rotate_impl(x, idx_ij, theta, scales, group_size):
     xc, idc, thc, scc, rows, h, krot = _rotate_args(x, idx_ij, theta, scales)
     dev = x.device
     out = torch.empty_like(xc)
-    if rows >= _PACKED_MIN_ROWS and rows * h < _PACKED_MAX_ELEMS:
+    if rows >= _PACKED_MIN_ROWS and rows * h < _packed_max_elems(krot, False):
         packed = _packed_for(idx_ij, theta, scales if scc is not None else None, group_size)
         if packed is not None:
             _rotate_rows(xc, packed, out, None, rows, h, krot, _lib.PQ_ROWS_SAME, "rotation::rotate")
@@ -288,7 +293,7 @@ def _rotate_mxfp4_impl(x, idx_ij, theta, scales, group_size):
     dev = x.device
     q = torch.empty((*x.shape[:-1], h // 2), dtype=torch.uint8, device=dev)
     sc = torch.empty((*x.shape[:-1], h // 32), dtype=torch.uint8, device=dev)
-    if rows >= _PACKED_MIN_ROWS and rows * h < _PACKED_MAX_ELEMS:
+    if rows >= _PACKED_MIN_ROWS and rows * h < _packed_max_elems(krot, True):
         packed = _packed_for(idx_ij, theta, scales if scc is not None else None, group_size)
         if packed is not None:
             _rotate_rows(xc, packed, q, sc, rows, h, krot, _lib.PQ_ROWS_MXFP4, "rotation::rotate_and_quant_mxfp4")

@@ -15,16 +15,20 @@ def to_np(t: torch.Tensor) -> np.ndarray:
     return t.numpy()
 
 
-def gemm_instances(fn):
-    """(name, template arguments) of the GEMM kernels that one call of fn launches, in launch order."""
+def kernel_instances(fn, pattern):
+    """(name, template arguments) of the kernels with names of the pattern that one call of fn launches, in order."""
     from torch.profiler import ProfilerActivity, profile
     fn()
     torch.cuda.synchronize()
     with profile(activities=[ProfilerActivity.CUDA]) as prof:
         fn()
         torch.cuda.synchronize()
-    found = [re.search(r"(gemm_\w+|w16_\w+)<([^>]*)>", e.name) for e in prof.events()]
+    found = [re.search(rf"\b({pattern})<([^>]*)>", e.name) for e in prof.events()]
     return [(m[1], tuple(a.strip() for a in m[2].split(","))) for m in found if m]
+
+
+def gemm_instances(fn):
+    return kernel_instances(fn, r"gemm_\w+|w16_\w+")
 
 
 def rel_fro(a, b) -> float:

@@ -1,4 +1,5 @@
-"""rotation::rotate and rotate_and_quant_mxfp4 from 4 M elements (the register chain derived on the device) against the
+"""rotation::rotate and rotate_and_quant_mxfp4 from 4 M elements (the register chain derived on the device; one and two
+layers without codes from 6 M) against the
 tile kernel that fewer run: the same float32 sequence, so the same bits, for every layer count, group size, odd row
 slice and the 64-channel tail; also for indices that pair no proper matching, and for blocks with NaN and infinities."""
 
@@ -9,7 +10,7 @@ import pytest
 import torch
 
 import alpamayo_amd  # noqa: F401
-from tests.gpu_util import to_np
+from tests.gpu_util import kernel_instances, to_np
 from tests.test_gpu_rotate import DT, _params
 
 pytestmark = pytest.mark.gpu
@@ -33,7 +34,9 @@ def _both(x, pairs, th, sc, gs):
 @pytest.mark.parametrize("dt", ["f32", "f16", "bf16"])
 @pytest.mark.parametrize("gs,krot,h,rows", [(128, 8, 256, 16385), (64, 1, 64, 65601), (64, 2, 192, 21900),
                                             (128, 4, 384, 10931), (64, 16, 320, 13113), (128, 8, 4096, 1027),
-                                            (128, 16, 128, 32773)])
+                                            (128, 16, 128, 32773),
+                                            # one and two layers without MXFP4 codes: from 6 M elements
+                                            (64, 1, 64, 93761), (64, 2, 192, 31261), (128, 2, 640, 9379)])
 @pytest.mark.parametrize("with_scale", [True, False])
 def test_chain_equals_tile(dt, gs, krot, h, rows, with_scale):
     print(f"chain dt={dt} gs={gs} krot={krot} h={h} rows={rows} scale={with_scale}", flush=True)
@@ -42,6 +45,34 @@ def test_chain_equals_tile(dt, gs, krot, h, rows, with_scale):
     x = torch.from_numpy(rng.standard_normal((rows, h)).astype(np.float32) * 3).to(DT[dt]).cuda()
     sc = torch.from_numpy(scales).to(DT[dt]).reshape(1, h).cuda() if with_scale else None
     _both(x, torch.from_numpy(pairs).cuda(), torch.from_numpy(theta).to(DT[dt]).cuda(), sc, gs)
+
+
+@pytest.mark.parametrize("krot,rows,h,chain,mx_chain", [
+    (8, 1024, 4096, True, True), (8, 1023, 4096, False, False), (1, 1024, 4096, False, True), (2, 1465, 4096, True, True),
+    (8, 31, 262144, False, False), (8, 32, 262144, True, True), (16, 1, 1 << 22, False, False),
+])
+def test_form_by_size(krot, rows, h, chain, mx_chain):
+    """The chain where every workgroup has a step of rows for it and the launch is large, else the tile form."""
+    print(f"form krot={krot} {rows}x{h}", flush=True)
+    x = torch.randn(rows, h, device="cuda").half()
+    pairs = torch.arange(128, dtype=torch.int16).repeat(krot, h // 128).cuda()
+    th = torch.rand(krot, h // 2, device="cuda").half()
+    for op, want in ((torch.ops.rotation.rotate, chain), (torch.ops.rotation.rotate_and_quant_mxfp4, mx_chain)):
+        found = kernel_instances(lambda: op(x, pairs, th, None, 128), r"rotate_\w+")   # noqa: B023
+        assert [f[0] for f in found] == ["rotate_chain" if want else "rotate_kernel"]
+
+
+@pytest.mark.parametrize("krot,rows,h,chain", [
+    (8, 192, 4096, True), (8, 191, 4096, False), (8, 31, 65536, False), (8, 32, 65536, True), (4, 1, 1 << 20, False),
+    (16, 47, 65536, False), (16, 48, 65536, True), (16, 300, 4096, False),
+])
+def test_backward_form_by_size(krot, rows, h, chain):
+    print(f"backward form krot={krot} {rows}x{h}", flush=True)
+    x, gy = torch.randn(2, rows, h, device="cuda").unbind(0)
+    pairs = torch.arange(128, dtype=torch.int16).repeat(krot, h // 128).cuda()
+    th = torch.rand(krot, h // 2, device="cuda")
+    found = kernel_instances(lambda: torch.ops.paroquant.rotate_backward(gy, x, pairs, th, None, 128), "rotate_chain_bwd")
+    assert [f[1][3] for f in found] == [str(chain).lower()]
 
 
 def test_special_values_and_fixed_layers():
