@@ -43,6 +43,7 @@ from typing import NamedTuple
 
 import torch
 import torch.nn as nn
+from torch.autograd.forward_ad import unpack_dual
 
 from .. import ops as _ops
 from .qmodule import WQLinear, unpack_intweight
@@ -176,7 +177,7 @@ class SharedInputRotateLinears(nn.Module):
         if self.w4a16:
             mode = None if norm_weight is None and residual is None else (
                 _ops._lib.PQ_PRO_ADD if norm_weight is None else _ops._lib.PQ_PRO_RMSNORM)
-            if mode is not None and self._fusable(x, residual, norm_weight) and 0.0 <= eps < 1.0:
+            if mode is not None and self._fusable(x, residual, norm_weight, eps):
                 w = norm_weight.to(x.dtype) if norm_weight is not None else None
                 return tuple(torch.ops.paroquant.w4a16_linear_group(x, *self._args(x), mode, residual, w, float(eps),
                                                                     return_normed, return_sum))
@@ -199,22 +200,28 @@ class SharedInputRotateLinears(nn.Module):
         return tuple(outs)
 
     @staticmethod
-    def _fusable(x, other, norm_weight=None):
+    def _fusable(x, other, norm_weight=None, eps=0.0):
         """Whether an elementwise step on x (and other) can run inside the rotation launch: same-shaped operands
-        of one type on one device, one weight per channel, and nothing to differentiate (the torch operations
-        that stand in otherwise broadcast, promote and record gradients).  Not while compiling: inductor makes
-        one kernel of the step by itself, with roundings of its own."""
+        of one type on one device, one weight per channel, an eps that the kernel takes, and nothing to differentiate
+        (the torch operations that stand in otherwise broadcast, promote, take numbers and record gradients and
+        tangents).  Not while compiling: inductor makes one kernel of the step by itself, with roundings of its own."""
         if torch.compiler.is_compiling():
             return False
-        for t in (other, norm_weight):
-            if t is not None and (t.device != x.device or not t.is_floating_point()):
+        operands = [t for t in (x, other, norm_weight) if t is not None]
+        for t in operands:
+            if not isinstance(t, torch.Tensor) or t.device != x.device or not t.is_floating_point():
                 return False
         if other is not None and (other.shape != x.shape or other.dtype != x.dtype):
             return False
-        if norm_weight is not None and norm_weight.numel() != x.size(-1):
-            return False
-        return x.dtype in _ops._DT and not (torch.is_grad_enabled() and any(
-            t is not None and t.requires_grad for t in (x, other, norm_weight)))
+        if norm_weight is not None:
+            k = x.size(-1)
+            if norm_weight.numel() != k or norm_weight.dim() > x.dim() or (k > 1 and norm_weight.size(-1) != k):
+                return False
+            # at most the largest float32 below one, which is what the kernel is given
+            if not isinstance(eps, (int, float)) or not 0.0 <= eps <= 1.0 - 2.0 ** -24:
+                return False
+        return x.dtype in _ops._DT and not (torch.is_grad_enabled() and any(t.requires_grad for t in operands)) \
+            and all(unpack_dual(t).tangent is None for t in operands)
 
     def forward_swiglu(self, gate: torch.Tensor, up: torch.Tensor, return_act: bool = False):
         """The members' outputs on act = silu(gate) * up in the inputs' dtype (a gated MLP's down_proj

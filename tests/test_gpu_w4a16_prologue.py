@@ -80,3 +80,36 @@ def test_module_operands_off_the_fused_path(m):
     xg = x.clone().requires_grad_(True)
     out = grp(xg, residual=r, norm_weight=w, return_normed=True, return_sum=True)
     assert out[-1].requires_grad and out[-2].requires_grad
+
+
+@pytest.mark.parametrize("m", [1, 40])
+def test_module_operands_torch_shapes(m):
+    """Weights, residuals and eps that torch's operations take in a form of their own: one more leading dimension, a
+    column, a number, an eps on the device, one that float32 rounds up to 1, and tangents of forward-mode AD."""
+    from torch.autograd import forward_ad
+
+    from alpamayo_amd.quantization import RotateLinearInt4, SharedInputRotateLinears
+    k, g = 1152, workloads.generator(9300)
+    rls = [RotateLinearInt4(k, 64, bias=False, dtype=torch.float16).cuda() for _ in range(2)]
+    for rl in rls:
+        rl.qlinear.scales.copy_(0.01 * torch.rand(rl.qlinear.scales.shape))
+    grp = SharedInputRotateLinears(rls)
+    x, r, t = (workloads.activations(m, k, g).half().cuda() for _ in range(3))
+    w = (0.8 + 0.4 * torch.rand(k, generator=g)).half().cuda()
+    w3, near1, eps_t = w.view(1, 1, k), 1.0 - 2.0 ** -30, torch.full((), 1e-6, device="cuda")
+    for got, rows in ((grp(x, norm_weight=w3), _rmsnorm_like_module(x, w3, 1e-6)),
+                      (grp(x, residual=r, norm_weight=w3), _rmsnorm_like_module(x + r, w3, 1e-6)),
+                      (grp(x, norm_weight=w, eps=near1), _rmsnorm_like_module(x, w, near1)),
+                      (grp(x, norm_weight=w, eps=eps_t), _rmsnorm_like_module(x, w, eps_t)),
+                      (grp(x, residual=0.5), x + 0.5),
+                      (grp.forward_swiglu(x, 0.5), torch.nn.functional.silu(x) * 0.5)):
+        for y, yp in zip(got, grp(rows)):
+            assert y.shape == yp.shape and torch.equal(y, yp)
+    if m > 1:
+        with pytest.raises(RuntimeError):
+            grp(x, norm_weight=w.view(k, 1))
+    with forward_ad.dual_level():
+        xd = forward_ad.make_dual(x, t)
+        assert forward_ad.unpack_dual(grp(xd, residual=r, return_sum=True)[-1]).tangent is not None
+        act = grp.forward_swiglu(xd, r, return_act=True)[-1]
+        assert forward_ad.unpack_dual(act).tangent is not None
