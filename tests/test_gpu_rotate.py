@@ -129,7 +129,12 @@ _BWD_TOL = {"f32": 2e-6, "f16": 2e-3, "bf16": 1.6e-2}
 @pytest.mark.parametrize("dt", ["f32", "f16", "bf16"])
 @pytest.mark.parametrize("gs,krot,h,rows", [(128, 8, 4096, 5), (128, 1, 256, 1), (64, 4, 192, 33),
                                             (128, 16, 384, 9), (64, 8, 64, 3), (128, 2, 1024, 3000),
-                                            (128, 8, 12288, 17), (64, 16, 320, 1030), (128, 8, 256, 0)])
+                                            (128, 8, 12288, 17), (64, 16, 320, 1030), (128, 8, 256, 0),
+                                            # past the sizes from which the register chain runs: every layer count,
+                                            # both group sizes, the 64-channel tail, rows that fill no last step
+                                            (128, 8, 256, 3101), (64, 8, 192, 4099), (64, 16, 320, 6557),
+                                            (64, 1, 64, 12301), (128, 4, 384, 2051), (128, 16, 128, 16411),
+                                            (64, 2, 1088, 727), (128, 8, 24704, 33)])
 @pytest.mark.parametrize("with_scale", [True, False])
 def test_rotate_backward_matches_oracle(dt, gs, krot, h, rows, with_scale):
     """paroquant::rotate_backward (one kernel pass + a fixed-order reduction) against the float64 oracle on
