@@ -59,32 +59,6 @@ constexpr int kept(int wk) { return wk >= 8 ? wk / 2 : wk; }
 template <int RB, int NT, int WK, int WN>
 constexpr size_t lds_bytes() { return static_cast<size_t>(kept(WK)) * WN * RB * NT * 4 * 64 * sizeof(float); }
 
-// Steps 0 .. n - 1 (n >= 1) of load and compute on two register stages, loads
-// two steps ahead; the tail is peeled so that no load sits behind a branch
-// (the compiler would wait for every load at the join).
-template <typename S, typename L, typename C>
-__device__ __forceinline__ void walk(int n, const L& load, const C& compute) {
-  S s0, s1;
-  load(s0, 0);
-  load(s1, min(1, n - 1));
-  int i = 0;
-  for (; i + 3 < n; i += 2) {
-    compute(s0, i);
-    load(s0, i + 2);
-    compute(s1, i + 1);
-    load(s1, i + 3);
-  }
-  if (n - i == 3) {
-    compute(s0, i);
-    load(s0, i + 2);
-    compute(s1, i + 1);
-    compute(s0, i + 2);
-  } else {
-    compute(s0, i);
-    if (n - i == 2) compute(s1, i + 1);
-  }
-}
-
 // grid: row tiles x column units (units of NT * WN 16-column tiles; members
 // start on a unit).  NTW: the weights are read by one row tile only, so they
 // are loaded non-temporally.
@@ -184,10 +158,30 @@ __global__ __launch_bounds__(WK * WN * 64) void gemm_mid(const pq::GemmGroup grp
     }
   };
 
-  // Wave wk walks the groups of its part of K (the host keeps WK <= G).
-  const int gb = wk * G / WK;
-  walk<Stage<RB, NT>>((wk + 1) * G / WK - gb, [&](Stage<RB, NT>& s, int i) { load(s, gb + i); },
-                      [&](const Stage<RB, NT>& s, int i) { compute(s, gb + i); });
+  // Wave wk walks the n groups of its part of K (the host keeps WK <= G).
+  // Two register stages; the tail is peeled so that no load sits behind a
+  // branch (the compiler would wait for every load at the join).
+  const int gb = wk * G / WK, n = (wk + 1) * G / WK - gb;
+  auto grp_of = [&](int i) { return gb + i; };
+  Stage<RB, NT> s0, s1;
+  load(s0, grp_of(0));
+  load(s1, grp_of(min(1, n - 1)));
+  int i = 0;
+  for (; i + 3 < n; i += 2) {
+    compute(s0, grp_of(i));
+    load(s0, grp_of(i + 2));
+    compute(s1, grp_of(i + 1));
+    load(s1, grp_of(i + 3));
+  }
+  if (n - i == 3) {
+    compute(s0, grp_of(i));
+    load(s0, grp_of(i + 2));
+    compute(s1, grp_of(i + 1));
+    compute(s0, grp_of(i + 2));
+  } else {
+    compute(s0, grp_of(i));
+    if (n - i == 2) compute(s1, grp_of(i + 1));
+  }
   if constexpr (PARTIALS) return;
 
   // Partial sums: red[wk][wn][(b, nt, v)][lane]

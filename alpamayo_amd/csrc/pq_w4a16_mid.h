@@ -24,6 +24,32 @@ constexpr int kParts16 = 8;
 template <int RB, int NT, int WN>
 constexpr size_t lds_bytes16() { return static_cast<size_t>(kParts16) * WN * RB * NT * 4 * 64 * sizeof(float); }
 
+// Steps 0 .. n - 1 (n >= 1) of load and compute on two register stages, loads
+// two steps ahead; the tail is peeled so that no load sits behind a branch
+// (the compiler would wait for every load at the join).
+template <typename S, typename L, typename C>
+__device__ __forceinline__ void walk(int n, const L& load, const C& compute) {
+  S s0, s1;
+  load(s0, 0);
+  load(s1, min(1, n - 1));
+  int i = 0;
+  for (; i + 3 < n; i += 2) {
+    compute(s0);
+    load(s0, i + 2);
+    compute(s1);
+    load(s1, i + 3);
+  }
+  if (n - i == 3) {
+    compute(s0);
+    load(s0, i + 2);
+    compute(s1);
+    compute(s0);
+  } else {
+    compute(s0);
+    if (n - i == 2) compute(s1);
+  }
+}
+
 template <int RB, int NT>
 struct Stage16 {
   v8h a[RB][4];
@@ -123,7 +149,7 @@ __global__ __launch_bounds__(WK * WN * 64, WK * WN == 4 ? 3 : 2) void w16_mid(co
 #pragma unroll
       for (int nt = 0; nt < NT; ++nt) acc[b][nt] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
     walk<Stage16<RB, NT>>((part + 1) * G / kParts16 - gb, [&](Stage16<RB, NT>& s, int i) { load(s, gb + i); },
-                          [&](const Stage16<RB, NT>& s, int) { compute(s); });
+                          compute);
     put(part);
   }
   __syncthreads();
