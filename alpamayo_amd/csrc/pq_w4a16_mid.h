@@ -7,9 +7,11 @@
 // instructions per 16 columns and group, is what RB rows blocks share.
 //
 // A row's outputs are the same bits in every configuration, so that a group of
-// linears returns what its members return alone: K falls into kParts16 parts,
-// a wave walks one of them or two neighbours, every part's sum starts from zero
-// and goes to LDS, and there the parts are added in one order.
+// linears returns what its members return alone: part p of K is every
+// kParts16-th group from group p on, a wave walks one part or two, every part's
+// sum starts from zero and goes to LDS, and there the parts are added in one
+// order.  (Contiguous parts, as in the W4A8 kernel, keep a workgroup's waves
+// further apart in A and took 1 to 4 % longer on a decoder layer's linears.)
 #pragma once
 
 #include "pq_gemm_mid.h"
@@ -58,7 +60,10 @@ struct Stage16 {
 };
 
 // (bounds of the 4-wave instance: three workgroups per CU)
-template <int RB, int NT, int WK, int WN>
+// FEW: fewer than two groups of K in some parts (K < 2048), where walk would load a lone group twice and a wave's second
+// part would start with nothing in flight: N = 4096, K = 1024, M = 400 21.9 -> 17.9 us with the rotation, K = 1536 23.9 ->
+// 22.7.  An instance of its own, because the branch costs the larger ones registers (4 x 2 blocks 5 % at K = 4096).
+template <int RB, int NT, int WK, int WN, bool FEW>
 __global__ __launch_bounds__(WK * WN * 64, WK * WN == 4 ? 3 : 2) void w16_mid(const W16Group grp, int bias_dtype, int y_dtype, int M, int K) {
   extern __shared__ __attribute__((aligned(16))) float red[];
   const int G = K >> 7;
@@ -138,19 +143,47 @@ __global__ __launch_bounds__(WK * WN * 64, WK * WN == 4 ? 3 : 2) void w16_mid(co
 #pragma unroll
         for (int v = 0; v < 4; ++v) dst[((b * NT + nt) * 4 + v) * 64] = acc[b][nt][v];
   };
-  // Wave wk walks parts wk PW .. wk PW + PW - 1, one after the other (the host keeps kParts16 <= G).  One loop over
-  // both, with the sum put away in its middle, costs the 4-wave instance its third wave per SIMD.
-  constexpr int PW = kParts16 / WK;
-#pragma unroll 1
-  for (int part = wk * PW; part < (wk + 1) * PW; ++part) {
-    const int gb = part * G / kParts16;
+  auto zero = [&] {
 #pragma unroll
     for (int b = 0; b < RB; ++b)
 #pragma unroll
       for (int nt = 0; nt < NT; ++nt) acc[b][nt] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
-    walk<Stage16<RB, NT>>((part + 1) * G / kParts16 - gb, [&](Stage16<RB, NT>& s, int i) { load(s, gb + i); },
-                          compute);
-    put(part);
+  };
+  // Wave wk walks parts wk, wk + WK, .. one after the other (the host keeps kParts16 <= G).  One loop over both of a
+  // 4-wave instance, with the sum put away in its middle, costs it its third wave per SIMD.
+  if constexpr (!FEW) {
+#pragma unroll 1
+    for (int part = wk; part < kParts16; part += WK) {
+      zero();
+      walk<Stage16<RB, NT>>((G - part + kParts16 - 1) / kParts16,
+                            [&](Stage16<RB, NT>& s, int i) { load(s, part + i * kParts16); }, compute);
+      put(part);
+    }
+  } else if (2 * WK == kParts16 && G == kParts16) {   // one group a part: both parts' loads first
+    Stage16<RB, NT> s0, s1;
+    load(s0, wk);
+    load(s1, wk + WK);
+    zero();
+    compute(s0);
+    put(wk);
+    zero();
+    compute(s1);
+    put(wk + WK);
+  } else {
+#pragma unroll 1
+    for (int part = wk; part < kParts16; part += WK) {
+      Stage16<RB, NT> s0, s1;
+      load(s0, part);
+      zero();
+      if (part + kParts16 < G) {
+        load(s1, part + kParts16);
+        compute(s0);
+        compute(s1);
+      } else {
+        compute(s0);
+      }
+      put(part);
+    }
   }
   __syncthreads();
   constexpr int CH = 4 * NT * WN;   // 4-column chunks per row
@@ -200,7 +233,11 @@ void launch_w16_mid_t(W16Group grp, int bias_dtype, int y_dtype, int M, int K, h
   for (int i = 0; i < grp.count; ++i) grp.first[i + 1] = grp.first[i] + (grp.mem[i].n / 16 + NT * WN - 1) / (NT * WN);
   const int nrt = ((M + 15) / 16 + RB - 1) / RB;
   const unsigned grid = static_cast<unsigned>(grp.first[grp.count]) * static_cast<unsigned>(nrt);
-  w16_mid<RB, NT, WK, WN><<<grid, WK * WN * 64, lds_bytes16<RB, NT, WN>(), stream>>>(grp, bias_dtype, y_dtype, M, K);
+  const size_t lds = lds_bytes16<RB, NT, WN>();
+  if (K < 2 * kParts16 * 128)
+    w16_mid<RB, NT, WK, WN, true><<<grid, WK * WN * 64, lds, stream>>>(grp, bias_dtype, y_dtype, M, K);
+  else
+    w16_mid<RB, NT, WK, WN, false><<<grid, WK * WN * 64, lds, stream>>>(grp, bias_dtype, y_dtype, M, K);
 }
 
 }  // namespace pqmid

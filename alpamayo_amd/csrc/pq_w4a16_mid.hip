@@ -1,4 +1,6 @@
 // Configuration and launch of the mid-size W4A16 GEMM (kernel: pq_w4a16_mid.h).
+#include <algorithm>
+
 #include "pq_w4a16_mid.h"
 
 namespace {
@@ -7,9 +9,12 @@ namespace {
 // a round of `slots` workgroups (the most the chip holds at once), fitted to
 // launches of one full round at K = 4096 (M = 64, 96, 128, 200, 512 at N = 4096:
 // 7.7, 9.3, 11.6, 17.7 and 29.5 us, 4.2 us of each fixed).  Small workgroups
-// replace each other as they finish, so theirs is paid in part rounds; their
-// waves walk two parts of K each, whose second starts with nothing in flight
-// (two groups' worth; K = 1024 1.25 times the time, K = 4096 1.03).
+// replace each other as they finish, so theirs is paid in part rounds (a fifth
+// at least: N = 2 x 6912, K = 4096, M = 33 26.5 us, 22.6 on 3 x 2 blocks), and
+// while the fp16 rows fit an XCD's L2 (4 MB: 2 M values) it is 0.83 of what it
+// is past that (with the rotation, N = 4096: M = 320, K = 4096 35.2 us against
+// 38.6 on eight waves of 2 x 2 blocks; M = 400, K = 12288 108 against 102 on
+// the 4 x 2 blocks in two columns).
 struct Cfg {
   int rb, nt, wk, wn, cost, slots;
   bool parts;
@@ -17,7 +22,7 @@ struct Cfg {
 constexpr Cfg kCfgs[] = {
     {2, 1, 8, 1, 60, 256, false},  {2, 2, 8, 1, 87, 256, false},  {2, 4, 8, 1, 170, 256, false},
     {3, 2, 8, 1, 127, 256, false}, {4, 2, 8, 1, 165, 256, false}, {4, 2, 4, 2, 330, 256, false},
-    {2, 2, 4, 1, 260, 768, true},
+    {2, 2, 4, 1, 215, 768, true},
 };
 
 struct Choice {
@@ -34,9 +39,11 @@ Choice choose(const int* n, int count, int m, int k) {
     int64_t units = 0;
     for (int q = 0; q < count; ++q) units += (n[q] / 16 + c.nt * c.wn - 1) / (c.nt * c.wn);
     const int64_t wgs = units * ((nrb + c.rb - 1) / c.rb);
-    double cost = c.cost * (c.parts ? static_cast<double>(wgs < c.slots ? c.slots : wgs) / c.slots
-                                    : static_cast<double>((wgs + c.slots - 1) / c.slots));
-    if (c.wk < pqmid::kParts16) cost *= 1.0 + 256.0 / k;
+    double rounds = static_cast<double>((wgs + c.slots - 1) / c.slots);
+    if (c.parts && wgs > c.slots && wgs % c.slots != 0)
+      rounds = static_cast<double>(wgs / c.slots) + std::max(static_cast<double>(wgs % c.slots) / c.slots, 0.2);
+    double cost = c.cost * rounds;
+    if (c.parts && static_cast<int64_t>(m) * k > 2 << 20) cost *= 1.2;
     if (i == 0 || cost < best.cost) best = {i, cost};
   }
   return best;
@@ -55,7 +62,7 @@ namespace pqw16 {
 bool w16_mid_takes(int64_t m, int64_t n, int64_t k) {
   if (m <= 16 || m > 512 || k < 1024) return false;
   const int two[2] = {static_cast<int>(n), static_cast<int>(n)};
-  const double per_cost = 0.00118 * static_cast<double>(k / 128) + 0.021;
+  const double per_cost = (k < 2048 ? 0.8 : 1.0) * (0.00118 * static_cast<double>(k / 128) + 0.021);   // FEW below 2048
   const double here = choose(two, 1, static_cast<int>(m), static_cast<int>(k)).cost * per_cost;
   const double here2 = choose(two, 2, static_cast<int>(m), static_cast<int>(k)).cost * per_cost;
   const double there = w16_prefill_us(m, n, k);

@@ -28,6 +28,9 @@ def _operands(n, K, seed, with_bias):
     (17, 1024, (16,)), (31, 1152, (1040,)), (33, 4096, (4096, 1024, 1024)), (48, 12288, (4096,)), (64, 1408, (12288, 12304)),
     (65, 4096, (4096,)), (97, 2048, (1040, 80)), (129, 4224, (4096,)), (200, 1024, (5120,)), (255, 1152, (4112,)),
     (320, 2048, (4096,)), (512, 1024, (4096, 1040)), (511, 1024, (272,)),
+    # every size of block with one, one or two, and more groups of K per part
+    (17, 1024, (8208,)), (30, 1920, (12304,)), (30, 2048, (8208,)), (33, 1024, (4096, 1040)), (47, 1920, (3856, 3840)),
+    (49, 1024, (4096, 1040)), (63, 1920, (4112,)), (49, 2176, (3856, 3840)), (511, 4224, (2064,)),
 ])
 def test_tiled_w16_gemm(M, K, ns):
     print(f"tiled W4A16 M={M} K={K} ns={ns}", flush=True)
@@ -56,6 +59,9 @@ def test_tiled_w16_gemm(M, K, ns):
 @pytest.mark.parametrize("M,K,ns", [
     (17, 1152, (4096, 1040)),
     (33, 1024, (12288, 12304)),          # one group per part of K, on both widths of workgroup
+    (33, 1024, (4096, 1040)),
+    (49, 1920, (3856, 3840)),            # parts of one and two groups
+    (49, 2176, (3856, 3840)),
     (48, 2176, (9728, 9728)),            # 17 groups: parts of two and three
     (64, 1152, (12288, 12288)),          # a lone member this wide asks for another split of K than the pair
     (65, 1024, (16, 8192)),
