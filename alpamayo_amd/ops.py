@@ -16,13 +16,13 @@ the ``paroquant`` namespace:
                          input_fp16, materialize_fp16, out_dtype) -> y
   paroquant::w4a8_linear_group(x, rot_idx[], rot_cs[], scales?[], krot, wpack[], wmeta[], bias?[],
                                input_fp16, materialize_fp16, out_dtype) -> y[]
-      (1..4 linears sharing the input x, in two launches for the whole group)
+      (1..4 linears sharing the input x, in the launches of one: one rotation, one GEMM)
   paroquant::w4a16_linear_group(x, <rotation and weight lists>, input_fp16, out_dtype, mode=0, x2=None,
                                 norm_weight=None, eps=0, return_h=False, return_sum=False) -> y[] (+ h) (+ x + x2)
       (the W4A16 group; with a mode behind a decoder layer's elementwise step, folded into its rotation launch)
   paroquant::w4a8_linear_group_rmsnorm(x, residual?, norm_weight, eps, <the group's arguments>,
                                        return_normed, return_sum) -> y[] (+ h) (+ x + residual)
-      (the same group behind a decoder layer's RMSNorm of x + residual, still two launches)
+      (the same group behind a decoder layer's RMSNorm of x + residual, in the same launches)
 
 ``pack_rotation`` (host) turns Rotation's pairs/angles into rot_idx/rot_cs;
 ``register_packed_rotation`` lets rotation::rotate find them (it never packs
@@ -125,7 +125,7 @@ class _DeviceGuard:
 
 
 def _same_device(name: str, t: torch.Tensor, dev: torch.device) -> None:
-    if not (t.device == dev):
+    if t.device != dev:
         raise RuntimeError(f"{name}: expected a tensor on {dev}, got {t.device}")
 
 
@@ -152,28 +152,28 @@ def linear_workspace_bytes(m: int, n: int, k: int, krot: int) -> int:
 
 def _rotate_args(x, idx_ij, theta, scales):
     """Checks of rotation::rotate's arguments; contiguous copies and the sizes."""
-    if not (x.dtype in _DT):
+    if x.dtype not in _DT:
         raise RuntimeError(f"rotate only supports Float, Half, and BFloat16, but got {x.dtype}")
-    if not (idx_ij.dtype == torch.int16):
+    if idx_ij.dtype != torch.int16:
         raise RuntimeError(f"idx_ij must be int16, got {idx_ij.dtype}")
-    if not (theta.dtype == x.dtype):
+    if theta.dtype != x.dtype:
         raise RuntimeError(f"theta must have x's dtype {x.dtype}, got {theta.dtype}")
-    if not (x.dim() >= 1 and x.size(-1) > 0):
+    if x.dim() < 1 or x.size(-1) <= 0:
         raise RuntimeError("x must have a non-empty last dimension")
     h = x.size(-1)
-    if not (idx_ij.dim() == 2 and theta.dim() == 2):
+    if idx_ij.dim() != 2 or theta.dim() != 2:
         raise RuntimeError("idx_ij and theta must be 2-D [KROT, H] / [KROT, H/2]")
     krot = theta.size(0)
-    if not (krot == idx_ij.size(0)):
+    if krot != idx_ij.size(0):
         raise RuntimeError("theta.size(0) must equal idx_ij.size(0)")
-    if not (idx_ij.size(1) == h and theta.size(1) * 2 == h):
+    if idx_ij.size(1) != h or theta.size(1) * 2 != h:
         raise RuntimeError(f"idx_ij must be [KROT, {h}] and theta [KROT, {h // 2}], got {tuple(idx_ij.shape)} / "
                            f"{tuple(theta.shape)}")
     has_scale = scales is not None and scales.numel() > 0
     if has_scale:
-        if not (scales.dtype == x.dtype):
+        if scales.dtype != x.dtype:
             raise RuntimeError(f"scales must have x's dtype {x.dtype}, got {scales.dtype}")
-        if not (scales.numel() == h):
+        if scales.numel() != h:
             raise RuntimeError(f"scales must hold {h} values, got {scales.numel()}")
     dev = x.device
     for nm, t in (("idx_ij", idx_ij), ("theta", theta)) + ((("scales", scales),) if has_scale else ()):
@@ -288,7 +288,7 @@ def _rotate_impl(x, idx_ij, theta, scales, group_size):
 
 def _rotate_mxfp4_impl(x, idx_ij, theta, scales, group_size):
     xc, idc, thc, scc, rows, h, krot = _rotate_args(x, idx_ij, theta, scales)
-    if not (h % 32 == 0):
+    if h % 32 != 0:
         raise RuntimeError(f"MXFP4 blocks are 32 channels: h={h}")
     dev = x.device
     q = torch.empty((*x.shape[:-1], h // 2), dtype=torch.uint8, device=dev)
@@ -327,7 +327,7 @@ def _rotate_mxfp4_fake(x, idx_ij, theta, scales, group_size):
 
 def _rotate_backward_impl(grad_y, x, idx_ij, theta, scales, group_size):
     xc, idc, thc, scc, rows, h, krot = _rotate_args(x, idx_ij, theta, scales)
-    if not (grad_y.shape == x.shape and grad_y.dtype == x.dtype):
+    if grad_y.shape != x.shape or grad_y.dtype != x.dtype:
         raise RuntimeError(f"grad_y must match x ({tuple(x.shape)}, {x.dtype}), got {tuple(grad_y.shape)}, "
                            f"{grad_y.dtype}")
     dev = x.device
@@ -375,7 +375,7 @@ def pack_rotation(pairs: torch.Tensor, cos_sin: torch.Tensor) -> tuple[torch.Ten
     p = pairs.detach().to("cpu", torch.int16).contiguous()
     cs = cos_sin.detach().to("cpu", torch.float32).contiguous()
     krot, h = p.shape
-    if not (cs.shape == (krot, h // 2, 2)):
+    if cs.shape != (krot, h // 2, 2):
         raise RuntimeError(f"cos_sin must be [{krot}, {h // 2}, 2]")
     sij, scs = packed_rotation_shapes(h, krot)
     rot_idx = torch.empty(sij, dtype=torch.int32)
@@ -389,11 +389,11 @@ def pack_rotation(pairs: torch.Tensor, cos_sin: torch.Tensor) -> tuple[torch.Ten
 
 def _check_rot_params(x, rot_idx, rot_cs, scales, krot):
     h = x.size(-1)
-    if not (x.dtype in _DT):
+    if x.dtype not in _DT:
         raise RuntimeError(f"x must be float32/float16/bfloat16, got {x.dtype}")
     if not (h % 128 == 0 and 0 < h <= 16384):
         raise RuntimeError(f"in_features={h} must be a multiple of 128 and <= 16384")
-    if not (1 <= krot <= 16):
+    if not 1 <= krot <= 16:
         raise RuntimeError(f"KROT={krot} must be in 1..16")
     sij, scs = packed_rotation_shapes(h, krot)
     if not (rot_idx.dtype in (torch.int32, torch.uint32) and rot_idx.shape == sij):
@@ -460,7 +460,7 @@ def _rotate_quant_rot_fake(x, rot_idx, rot_cs, scales, krot, input_fp16, materia
 
 
 def _quant_impl(x):
-    if not (x.dtype in _DT):
+    if x.dtype not in _DT:
         raise RuntimeError(f"x must be float32/float16/bfloat16, got {x.dtype}")
     h = x.size(-1)
     if not (h % 8 == 0 and h > 0):
@@ -503,7 +503,7 @@ def _check_weights(wpack, wmeta, dev):
 
 
 def _gemm_launch(xq, xs, wpack, wmeta, bias, out_dtype, m, n, k, dev):
-    if not (out_dtype in _DT):
+    if out_dtype not in _DT:
         raise RuntimeError(f"out_dtype must be float32/float16/bfloat16, got {out_dtype}")
     y = torch.empty((m, n), dtype=out_dtype, device=dev)
     if bias is not None:
@@ -609,10 +609,10 @@ def _prepack_fake(awq_qweight, awq_scales, awq_qzeros):
 def _linear_impl(x, rot_idx, rot_cs, scales, krot, wpack, wmeta, bias, input_fp16, materialize_fp16, out_dtype):
     dev = x.device
     n, k = _check_weights(wpack, wmeta, dev)
-    if not (x.size(-1) == k):
+    if x.size(-1) != k:
         raise RuntimeError(f"x has {x.size(-1)} features, the weights expect {k}")
     _check_rot_params(x, rot_idx, rot_cs, scales, krot)
-    if not (out_dtype in _DT):
+    if out_dtype not in _DT:
         raise RuntimeError(f"out_dtype must be float32/float16/bfloat16, got {out_dtype}")
     xc = x.contiguous()
     m = xc.numel() // k
@@ -647,11 +647,11 @@ def _group_members(x, rot_idx, rot_cs, scales, krot, wpack, wmeta, bias, out_dty
     """The pq_linear_member table of a group over x [.., k], the outputs it writes, and what must stay alive."""
     dev = x.device
     count = len(wpack)
-    if not (1 <= count <= _lib.MAX_GROUP):
+    if not 1 <= count <= _lib.MAX_GROUP:
         raise RuntimeError(f"a group holds 1..{_lib.MAX_GROUP} linears, got {count}")
-    if not (len(rot_idx) == len(rot_cs) == len(scales) == len(wmeta) == len(bias) == count):
+    if not len(rot_idx) == len(rot_cs) == len(scales) == len(wmeta) == len(bias) == count:
         raise RuntimeError("every per-member list must have one entry per linear")
-    if not (out_dtype in _DT):
+    if out_dtype not in _DT:
         raise RuntimeError(f"out_dtype must be float32/float16/bfloat16, got {out_dtype}")
     k = x.size(-1)
     m = x.numel() // k
@@ -659,7 +659,7 @@ def _group_members(x, rot_idx, rot_cs, scales, krot, wpack, wmeta, bias, out_dty
     keep, outs, bias_dt = [], [], 0
     for i in range(count):
         n, kw = _check_weights(wpack[i], wmeta[i], dev)
-        if not (kw == k):
+        if kw != k:
             raise RuntimeError(f"member {i}: the weights expect {kw} features, x has {k}")
         _check_rot_params(x, rot_idx[i], rot_cs[i], scales[i], krot)
         idx, cs = rot_idx[i].contiguous(), rot_cs[i].contiguous()
@@ -670,7 +670,7 @@ def _group_members(x, rot_idx, rot_cs, scales, krot, wpack, wmeta, bias, out_dty
                 raise RuntimeError(f"member {i}: bias must hold {n} float values")
             _same_device("bias", b, dev)
             b = b.contiguous()
-            if not (bias_dt in (0, _DT[b.dtype])):
+            if bias_dt not in (0, _DT[b.dtype]):
                 raise RuntimeError("all biases of a group must share one dtype")
             bias_dt = _DT[b.dtype]
         y = torch.empty((m, n), dtype=out_dtype, device=dev)
@@ -715,30 +715,30 @@ def _aligned16(t):
 def _prologue_args(x, x2, norm_weight, mode, return_h, return_sum):
     """Checks of a fused group's elementwise step; contiguous x, x2 and norm_weight."""
     dev = x.device
-    if not (x.dtype in _DT):
+    if x.dtype not in _DT:
         raise RuntimeError(f"x must be float32/float16/bfloat16, got {x.dtype}")
-    if not (mode in (_lib.PQ_PRO_RMSNORM, _lib.PQ_PRO_ADD, _lib.PQ_PRO_SWIGLU)):
+    if mode not in (_lib.PQ_PRO_RMSNORM, _lib.PQ_PRO_ADD, _lib.PQ_PRO_SWIGLU):
         raise RuntimeError(f"unknown prologue mode {mode}")
     xc = x.contiguous()
     k = xc.size(-1)
     w = None
     if mode == _lib.PQ_PRO_RMSNORM:
-        if not (norm_weight is not None and norm_weight.dtype == x.dtype and norm_weight.numel() == k):
+        if norm_weight is None or norm_weight.dtype != x.dtype or norm_weight.numel() != k:
             raise RuntimeError(f"norm_weight must hold {k} values of x's dtype {x.dtype}")
         _same_device("norm_weight", norm_weight, dev)
         w = norm_weight.contiguous()
     else:
-        if not (x2 is not None):
+        if x2 is None:
             raise RuntimeError("the add and the SwiGLU need x2 (residual / up)")
     other = None
     if x2 is not None:
-        if not (x2.shape == x.shape and x2.dtype == x.dtype):
+        if x2.shape != x.shape or x2.dtype != x.dtype:
             raise RuntimeError("x2 (residual / up) must match x's shape and dtype")
         _same_device("x2", x2, dev)
         other = x2.contiguous()
-    if not (not return_sum or (other is not None and mode != _lib.PQ_PRO_SWIGLU)):
+    if return_sum and (other is None or mode == _lib.PQ_PRO_SWIGLU):
         raise RuntimeError("return_sum needs a residual (RMSNorm with residual, or the add)")
-    if not (not return_h or mode != _lib.PQ_PRO_ADD):
+    if return_h and mode == _lib.PQ_PRO_ADD:
         raise RuntimeError("the add has no h: use return_sum")
     return xc, other, w
 
@@ -884,7 +884,7 @@ def w4a8_linear_group_intermediates(x, rot_idx, rot_cs, scales, krot, wpack, wme
     (codes int8 [count, m, k], xscale float32 [count, m], [partials int32 [m, k/128, n_i] per member],
     h or None, s or None)."""
     dev = x.device
-    if not (x.dtype in _DT):
+    if x.dtype not in _DT:
         raise RuntimeError(f"x must be float32/float16/bfloat16, got {x.dtype}")
     xc = x.contiguous()
     k = xc.size(-1)
@@ -973,11 +973,11 @@ def _w16_prepack_fake(awq_qweight, scales, scaled_zeros):
 def _w16_gemm_impl(x, wpack, wmeta, bias, out_dtype):
     dev = x.device
     n, k = _check_weights(wpack, wmeta, dev)
-    if not (x.dtype == torch.float16):
+    if x.dtype != torch.float16:
         raise RuntimeError(f"x must be float16 (the W4A16 kernels take fp16 activations), got {x.dtype}")
-    if not (x.size(-1) == k):
+    if x.size(-1) != k:
         raise RuntimeError(f"x has {x.size(-1)} features, the weights expect {k}")
-    if not (out_dtype in _DT):
+    if out_dtype not in _DT:
         raise RuntimeError(f"out_dtype must be float32/float16/bfloat16, got {out_dtype}")
     xc = x.contiguous()
     m = xc.numel() // k
@@ -1008,10 +1008,10 @@ def w4a16_linear_workspace_bytes(m: int, k: int) -> int:
 def _w16_linear_impl(x, rot_idx, rot_cs, scales, krot, wpack, wmeta, bias, input_fp16, out_dtype):
     dev = x.device
     n, k = _check_weights(wpack, wmeta, dev)
-    if not (x.size(-1) == k):
+    if x.size(-1) != k:
         raise RuntimeError(f"x has {x.size(-1)} features, the weights expect {k}")
     _check_rot_params(x, rot_idx, rot_cs, scales, krot)
-    if not (out_dtype in _DT):
+    if out_dtype not in _DT:
         raise RuntimeError(f"out_dtype must be float32/float16/bfloat16, got {out_dtype}")
     xc = x.contiguous()
     m = xc.numel() // k
@@ -1039,12 +1039,13 @@ _pq_lib.impl("w4a16_linear", _w16_linear_impl, "CUDA")
 
 def _w16_linear_group_impl(x, rot_idx, rot_cs, scales, krot, wpack, wmeta, bias, input_fp16, out_dtype, mode=0,
                            x2=None, norm_weight=None, eps=0.0, return_h=False, return_sum=False):
-    """paroquant::w4a16_linear for linears that read the same x, in one rotation launch and (m <= 16) one GEMM;
-    with a mode (PQ_PRO_*) behind that elementwise step, which runs inside the rotation launch."""
+    """paroquant::w4a16_linear for linears that read the same x, in one rotation launch and one GEMM launch (above 16
+    rows one for the members on the mid-size GEMM and one for each on the prefill tiles); with a mode (PQ_PRO_*) behind
+    that elementwise step, which runs inside the rotation launch."""
     dev = x.device
-    if not (x.dtype in _DT):
+    if x.dtype not in _DT:
         raise RuntimeError(f"x must be float32/float16/bfloat16, got {x.dtype}")
-    if not (mode != 0 or not (x2 is not None or norm_weight is not None or return_h or return_sum)):
+    if mode == 0 and (x2 is not None or norm_weight is not None or return_h or return_sum):
         raise RuntimeError("x2, norm_weight, return_h and return_sum need a mode")
     if mode:
         xc, other, w = _prologue_args(x, x2, norm_weight, mode, return_h, return_sum)
