@@ -157,8 +157,8 @@ PQ_HIDDEN void launch_gemm_group_partials(GemmGroup grp, int aq, int m, int k, h
 // Past 256 rows a wide launch is best on 192 x 256 tiles, which have no room for chains (gate and up, N = 24576, K =
 // 4096, M = 320: 72 us in one chain, 81 to 103 in four), so only short rows (small hidden sizes: few columns too; to
 // 384 rows) and long ones (down: N = 4096, K = 12288, M = 320: 71 us on the prefill tiles, 51 here) stay.
-// Two decoder layers in us, all sizes in one chain / by this rule, hidden 1536 / MLP 3840 M = 300 175 / 148, 4096 /
-// 12288 M = 300 474 / 422 (four chains for every K: 469).
+// Two decoder layers in us, all sizes in one chain / by this rule / four chains for every K: hidden 1536 / MLP 3840
+// M = 300 175 / 160 / 148, 4096 / 12288 M = 300 474 / 426 / 469.
 constexpr int kMidFixedRows = 64, kMidMaxRows = 512, kMidChains = 4;
 constexpr int gemm_mid_waves(int64_t m, int64_t k) {
   if (k < 1024 || m > (k >= 6144 ? kMidMaxRows : k <= 3072 ? 384 : 256)) return 0;

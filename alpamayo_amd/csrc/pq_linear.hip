@@ -11,11 +11,14 @@
 //     are already in flight.
 //   split3 (k >= 4096 beyond that, up to 64 tokens): the split rotation
 //     with the rows spread over waves, a token-scale + int8 kernel, then
-//     the decode GEMM on int8 A (three launches; from 17 rows the mid-size
-//     GEMM, for which the codes are written tiled).
+//     the GEMM on int8 A (three launches).
 //   rows (otherwise): pq_rotate_quant_i8 (rotation + absmax + int8 quant of
-//     whole rows per workgroup) into the caller's workspace, then the
-//     mid-size GEMM (17 to 512 rows) or the kernels of pq_w4a8_gemm.
+//     whole rows per workgroup) into the caller's workspace, then the GEMM
+//     on int8 A.
+//
+// The GEMM on int8 A is one of pq_w4a8_gemm's kernels or, at 17 to 512 rows
+// where it is faster (pq::gemm_mid_choice), the mid-size GEMM, for which the
+// codes are written tiled, or the prefill tiles in its order of the sum.
 //
 // A one-kernel variant (every workgroup rotating the token itself) was
 // measured slower: the K/128 x 5 KB of rotation parameters, re-read by each
@@ -51,7 +54,7 @@ bool use_split(int64_t m, int64_t k) {
 
 // Rows of 4096 channels or more past the split pair, up to 64 tokens: the
 // split rotation with its rows spread over waves (kSplitRowsPerWave rows
-// each), a small kernel for the token scales and int8 codes, then the decode
+// each), a small kernel for the token scales and int8 codes, then the
 // GEMM on int8 A.  The row kernel runs each row on one CU, whose VALU needs
 // about 12 us for the 96 groups of a 12288-channel row (down, k = 12288, at
 // m = 6: 17.8 us against 22.2 us; m = 16: 20.0 / 24.0).  At k = 4096 the

@@ -30,8 +30,8 @@
 //                fixed-order LDS sum of their partials), four
 //                v_mfma_f32_16x16x32_f16 per 1 KB weight block, A rows read
 //                from memory (rows past M repeat row M-1, never stored).
-//   w16_mid      17 to 512 rows behind the linear entry points, until the prefill
-//                tiles fill the chip: pq_w4a16_mid.h.
+//   w16_mid      17 to 512 rows behind the linear entry points, where it is
+//                estimated faster for the linear alone: pq_w4a16_mid.h.
 //   w16_prefill  M > 16: 192x256 (or 128x128) tiles, 8 (or 4) waves side by
 //                side along n, v_mfma_f32_32x32x16_f16.  A stage of the LDS
 //                ring is half a K group (64 k): BM rows x 128 B of A

@@ -101,14 +101,16 @@ class SharedInputRotateLinears(nn.Module):
     """Linears that read the same activation -- q/k/v, or gate/up -- run as one group.
 
     Each member keeps its own rotation and weights; forward(x) returns the
-    members' outputs, equal to calling each member on x.  Members are
+    members' outputs, equal to calling each member on x: bit for bit past 64
+    rows (W4A16: past 16), below within the rounding of another order of the
+    float32 sum over K.  Members are
     BF16RotateLinearWrapper or RotateLinearInt4 modules (all of one kind)
     with one in_features and one number of rotation layers, holding
-    MarlinW4A8Linear weights (W4A8: paroquant::w4a8_linear_group, one
-    rotation + quant launch for all members and one GEMM launch over their
-    concatenated output columns, where separate calls take two launches per
-    linear) or all WQLinear weights (W4A16: paroquant::w4a16_linear_group,
-    one rotation launch and, at decode and mid sizes, one GEMM launch).  The reference
+    MarlinW4A8Linear weights (W4A8: paroquant::w4a8_linear_group, the
+    rotation + quant launches of one linear for all members and one GEMM
+    launch over their concatenated output columns) or all WQLinear weights
+    (W4A16: paroquant::w4a16_linear_group, one rotation launch and, at decode
+    and mid sizes, one GEMM launch).  The reference
     keeps these linears separate once ParoQuant is loaded
     (paroquant_marlin_w4a8.py:455-460); its unquantised counterparts are
     QKVLinear / MergedColumnLinear (patches.py:144-263).
@@ -167,7 +169,7 @@ class SharedInputRotateLinears(nn.Module):
         x (+ residual): h = weight * (s * rsqrt(mean(s^2) + eps)) with s = x + residual, in x's dtype
         (Qwen3VLTextRMSNorm.forward, modeling_qwen3_vl.py:354-359); with only ``residual``, on
         s = x + residual (a decoder layer's residual add).  The norm runs inside the group's rotation
-        launch, and so does the add, except with W4A8 members past decode sizes (a separate torch add).
+        launch, and so does the add, except with W4A8 members that run the row rotation (a torch add there).
         ``return_normed`` / ``return_sum`` append h / s to the outputs."""
         if return_normed and norm_weight is None:
             raise ValueError("return_normed needs norm_weight (the add alone returns its sum: return_sum)")

@@ -214,7 +214,7 @@ int pq_w4a8_prepack(const int32_t* awq_qweight, const uint16_t* awq_scales,
  *   split pair (m*k <= 8192, or k >= 8192 and m <= 2): the rotated rows and
  *     per-group maxima, m*k*4 rounded up to 256 plus 4*m*(k/128) bytes;
  *   three launches (k a multiple of 128 in [4096, 16384], beyond the split
- *     pair, up to m = 32): both of those plus the int8 activations and
+ *     pair, up to m = 64): both of those plus the int8 activations and
  *     their scales (m*k rounded up to 256, plus 4*m);
  *   otherwise (the row rotate+quant kernel): the int8 activations and their
  *     scales only, m*k rounded up to 256 plus 4*m bytes.
@@ -224,7 +224,11 @@ size_t pq_w4a8_linear_workspace_size(int64_t m, int64_t n, int64_t k, int krot);
 /* y = W4A8 GEMM of the per-token int8 quantization of the rotation of x:
  * x [m, k] (x_dtype) -> y [m, n] (y_dtype), rotation operands as for
  * pq_rotate_quant_i8, weights as for pq_w4a8_gemm, flags PQ_RQ_*.
- * k <= 16384.  Same results as pq_rotate_quant_i8 followed by pq_w4a8_gemm.
+ * k <= 16384.  Same codes, scales and int32 partials as pq_rotate_quant_i8
+ * followed by pq_w4a8_gemm, and the same bits of y past 512 rows.  Below, the
+ * scaled partials may be added in another order, which follows from m and k
+ * past 64 rows and from m, k and the columns of the launch up to there: a
+ * row's y can differ in the float32 rounding between calls of another m.
  * Reference: paroquant_marlin_w4a8.py:59-65, 314-333; rotation_linear.py:120-124. */
 int pq_w4a8_linear(const void* x, int x_dtype, const uint32_t* rot_idx, const float* rot_cs, const float* scales,
                    const uint8_t* wpack, const uint32_t* wmeta, const void* bias, int bias_dtype, void* y,
@@ -272,11 +276,11 @@ typedef struct pq_linear_member {
  * over the chip): with a GEMM that quantizes A itself (m*k <= 8192,
  * or k >= 8192 and m <= 2), or for rows of 4096 channels or more (k a
  * multiple of 128 in [4096, 16384], up to 64 tokens) with a token-scale +
- * int8 kernel and the
- * GEMM on int8 A.  0 when they run the row rotate+quant kernel plus the
- * GEMM.  Callers use it to decide whether an elementwise step is cheaper
- * fused into the rotation launch (it is on the split path) or as a separate
- * kernel.  No counterpart in the reference. */
+ * int8 kernel and the GEMM on int8 A.  0 when they run the row rotate+quant
+ * kernel plus the GEMM.  Callers use it for the residual add alone, which is
+ * cheaper inside the rotation launch on the split path and as a kernel of its
+ * own otherwise (the norm and the gated activation are cheaper inside
+ * everywhere).  No counterpart in the reference. */
 int pq_w4a8_linear_split_path(int64_t m, int64_t k);
 
 /* Bytes of workspace pq_w4a8_linear_group needs for count members sharing an
@@ -285,9 +289,11 @@ int pq_w4a8_linear_split_path(int64_t m, int64_t k);
 size_t pq_w4a8_linear_group_workspace_size(int64_t m, int64_t k, int count);
 
 /* count (1..4) W4A8 linears over the same input x [m, k] (x_dtype), each with
- * its own rotation and weights: member i writes its y [m, n_i].  Same results
- * as pq_w4a8_linear per member, in two launches for the whole group -- one
- * rotation (+ quant) launch and one GEMM over the concatenated columns.
+ * its own rotation and weights: member i writes its y [m, n_i].  The results
+ * of pq_w4a8_linear per member -- bit for bit past 64 rows, below within the
+ * rounding of another order of the float32 sum over K -- in the rotation (+
+ * quant) launches of one linear and one GEMM over the concatenated columns
+ * (two where its leading members fill whole rounds of the chip).
  * All members share k, krot, flags, bias_dtype and y_dtype.  No counterpart
  * in the reference, whose ParoQuant loading runs q/k/v and gate/up as
  * separate linears (paroquant_marlin_w4a8.py:455-460); it replaces, for one
@@ -297,7 +303,7 @@ int pq_w4a8_linear_group(const void* x, int x_dtype, const pq_linear_member* mem
                          int y_dtype, int64_t m, int64_t k, int krot, unsigned flags, void* workspace,
                          size_t workspace_bytes, void* stream);
 
-/* pq_w4a8_linear_group behind a decoder layer's RMSNorm, in the same two
+/* pq_w4a8_linear_group behind a decoder layer's RMSNorm, in the same
  * launches: the members read h instead of x, where
  *   s = x + residual (rounded to x's dtype; s = x when residual is NULL),
  *   h = round(w * round(s * rsqrt(mean(s^2) + eps))),
@@ -345,7 +351,9 @@ size_t pq_w4a16_linear_workspace_size(int64_t m, int64_t k);
 
 /* y = pq_w4a16_gemm of the rotation of x, rounded to fp16: x [m, k]
  * (x_dtype f32/f16/bf16), rotation operands as for pq_w4a8_linear,
- * flags 0 or PQ_RQ_INPUT_FP16 (round x to fp16 first).  Two launches.
+ * flags 0 or PQ_RQ_INPUT_FP16 (round x to fp16 first).  Two launches.  At
+ * 17 to 512 rows the float32 sum over K may run in another order than
+ * pq_w4a16_gemm's, by m, n and k: the same value up to its rounding.
  * Reference: RotateLinearInt4.forward with a WQLinear qlinear
  * (rotation_linear.py:136-139): rotation::rotate (rotation.cu:456-493),
  * then WQLinear.forward (qmodule.py:207-232). */
@@ -381,7 +389,7 @@ int pq_w4a16_linear_group_fused(const void* x, const void* x2, const void* norm_
                                 void* workspace, size_t workspace_bytes, void* stream);
 
 /* pq_w4a8_linear_group behind a decoder layer's elementwise step, chosen by
- * mode (PQ_PRO_*), in the same two launches; the members read
+ * mode (PQ_PRO_*), in the same launches; the members read
  *   PQ_PRO_RMSNORM: h = RMSNorm(x + x2) exactly as pq_w4a8_linear_group_rmsnorm
  *                   (x2 = residual, may be NULL; norm_weight, eps as there);
  *   PQ_PRO_ADD:     s = x + x2 (rounded to x's dtype; x2 required);

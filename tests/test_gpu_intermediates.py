@@ -3,9 +3,9 @@
 The linear entry points pick one of three launch sequences by token count and row length: the split pair
 (split rotation, then a decode GEMM that derives the token scales and int8 codes itself: in registers at one
 and two tokens, into LDS otherwise),
-the three-launch long-row path (split rotation, quant_split_kernel, decode GEMM on int8 A) and the row
-rotate+quant kernel followed by the decode GEMM (up to 64 rows) or the prefill GEMM (tile-pair form on its big
-tiles).  The intermediates entry point runs the same launches with the GEMM in its partials form and returns the
+the three-launch long-row path (split rotation, quant_split_kernel, GEMM on int8 A) and the row rotate+quant
+kernel followed by the GEMM.  The GEMM on int8 A is the decode one, from 17 rows the mid-size one where it is
+faster, or the prefill GEMM (tile-pair form on its big tiles).  The intermediates entry point runs the same launches with the GEMM in its partials form and returns the
 int8 codes and token scales that GEMM used and its int32 per-group partials.  Checked here, against the oracle,
 for every path, every prologue (none, RMSNorm, residual add, SwiGLU), single linears and groups, on the
 Qwen3-8B decoder-layer shapes at 1-64 tokens and at prefill sizes:

@@ -98,7 +98,7 @@ def test_swiglu_group(M, K, ns):
 @pytest.mark.parametrize("M", [1, 16])
 def test_module_options_and_graph_replay(M):
     """SharedInputRotateLinears(x, residual=r) and .forward_swiglu(gate, up) inside a captured graph: fused
-    into the rotation at M = 1 (split path), separate torch ops at M = 16 (row path)."""
+    into the rotation in both (rows of 4096 channels run the split rotation to 64 tokens)."""
     K = 4096
     g = workloads.generator(4343)
     from alpamayo_amd.quantization import SharedInputRotateLinears
